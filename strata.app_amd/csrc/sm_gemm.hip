@@ -38,8 +38,9 @@ __device__ __forceinline__ uint32_t xcd_remap(uint32_t b, uint32_t real) {
 // and multiplied, the raw weight fragments and the activation chunk of slab sb+1 are
 // already in flight into registers; one LDS buffer holds the current activation slab.
 // FULL: K is a multiple of 256, so every load is unconditional and the loop has no
-// divergent branches; otherwise (Q8_0 widths that end mid-slab) lane groups past K load
-// from a clamped in-bounds address and contribute zero weights and activations.
+// divergent branches; otherwise (Q8_0 widths that end mid-slab) threads past K load the start
+// of their row instead (column 0, weight group 0: inside the row whatever K is) and contribute
+// zero weights and activations.
 template <class Frag, bool FULL>
 __device__ __forceinline__ void tile_mma(const _Float16* __restrict__ a_rows, uint32_t a0,
                                          uint32_t a_last, uint32_t K, uint32_t n_rb, const uint8_t* w0row,
@@ -55,16 +56,17 @@ __device__ __forceinline__ void tile_mma(const _Float16* __restrict__ a_rows, ui
     for (int i = 0; i < 8; ++i) {
         uint32_t row = a0 + r0 + 8 * i;
         if (row > a_last) row = a_last;
-        arow[i] = a_rows + uint64_t(row) * K + 8 * cc;
+        arow[i] = a_rows + uint64_t(row) * K;
     }
     const half8 zero{0, 0, 0, 0, 0, 0, 0, 0};
     half8 areg[8];
     Frag f0, f1;
     auto load_slab = [&](uint32_t sb) {
-        uint32_t ka = sb * kSlab, kb = sb;
+        uint32_t ka = sb * kSlab + 8u * cc, kb = sb;
+        int kg = g;
         if (!FULL) {
-            if (ka + 8u * cc >= K) ka = 0;             // clamped; zeroed below
-            if (sb * kSlab + 64u * g >= K) kb = 0;     // clamped; zeroed at decode time
+            if (ka >= K) ka = 0;                                        // zeroed below
+            if (sb * kSlab + 64u * g >= K) { kb = 0; kg = 0; }          // zeroed at decode time
         }
 #pragma unroll
         for (int i = 0; i < 8; ++i) areg[i] = *reinterpret_cast<const half8*>(arow[i] + ka);
@@ -72,8 +74,8 @@ __device__ __forceinline__ void tile_mma(const _Float16* __restrict__ a_rows, ui
 #pragma unroll
             for (int i = 0; i < 8; ++i) areg[i] = zero;
         }
-        f0.load(w0row + uint64_t(kb) * kSB, g);
-        f1.load(w1row + uint64_t(kb) * kSB, g);
+        f0.load(w0row + uint64_t(kb) * kSB, kg);
+        f1.load(w1row + uint64_t(kb) * kSB, kg);
     };
     load_slab(0);
     for (uint32_t sb = 0; sb < n_slabs; ++sb) {

@@ -116,3 +116,12 @@ def test_tile_broken_destination_zeroes_parts(moe, layer, orc, gpu_ctx, stream):
     _, _, st_dn = ws.read_status(stream)
     assert st_dn & 2
     assert (gu.host(ws.parts, np.float32) == 0).all()
+
+
+@pytest.mark.parametrize("ff", [64, 128, 192, 320])
+def test_short_reduction_rows(moe, layer, orc, gpu_ctx, stream, ff):
+    """Down reductions that end inside a 256-value slab: the lanes past K stay inside their row
+    (rows of 64 to 192 values are shorter than the slab that the other lanes cover)."""
+    print(f"case tiles short reduction {ff}", flush=True)
+    cfg = layer.LayerConfig("tiles_short", 96, 256, 12, 2, ff, 0, moe.Q8_0, moe.Q8_0, moe.F16, seed=311)
+    _check_layer(moe, layer, orc, gpu_ctx, stream, cfg)
