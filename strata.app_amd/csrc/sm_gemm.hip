@@ -316,7 +316,7 @@ hipError_t launch_staged(const RoutedGemm& g, hipStream_t s) {
     const TilePlan p = tile_plan<MODE, NF>(g.k, g.n_out);
     // Persistent: one workgroup per CU (each holds about 130 KB of LDS), never more than the
     // tile slots, in whole groups of 8 (one per XCD).
-    uint32_t blocks = (g.tile_capacity * p.n_chunks + 7u) & ~7u;
+    uint32_t blocks = (g.tile_capacity * p.n_ntiles + 7u) & ~7u;
     const uint32_t cap = device_cus() & ~7u;
     if (blocks > cap) blocks = cap;
     if (blocks < 8u) blocks = 8u;

@@ -405,9 +405,10 @@ struct DirectWeights {
 };
 
 // Launch shape of the staged tile kernels for one stage: column tiles of 128*NF weight rows,
-// `npi` of them per item (about 8 (column tile, slab) steps per item; with the activation tile
-// resident (K <= 512) every column tile of a row tile goes to one item, so the tile is read
-// once).
+// at most `npi` of them per item (about 8 (column tile, slab) steps per item; with the activation
+// tile resident (K <= 512) every column tile of a row tile goes to one item, so the tile is read
+// once); a stage of few row tiles splits further (split_npi). n_chunks: the slots of a row tile
+// that a failed plan check zeroes.
 struct TilePlan {
     uint32_t n_ntiles, npi, n_chunks;
     bool resident;
@@ -422,6 +423,17 @@ inline TilePlan tile_plan(uint32_t k, uint32_t n_out) {
     p.n_chunks = (p.n_ntiles + p.npi - 1) / p.npi;
     p.resident = n_slabs <= 2;
     return p;
+}
+
+// Column tiles per item for `tiles` row tiles on this grid: the launch's npi, halved while there
+// would be fewer items than workgroups. What few row tiles cost is then the longest item, not
+// bandwidth: 64 row tiles of 4 column tiles (d = 1024, I = 512) took 31.4 us as 64 down items and
+// 16.2 us as 256, and 128 row tiles of 8 (d = 2048, Q8_0) 65 -> 49 us. Past one item per
+// workgroup a split only re-reads activations: halving on to two items each measured 110.5 ->
+// 116 us (440 row tiles) and 49 -> 51 us (128), to four 175 -> 187 us (515).
+__device__ __forceinline__ uint32_t split_npi(uint32_t tiles, uint32_t n_ntiles, uint32_t npi) {
+    while (npi > 1u && tiles * ((n_ntiles + npi - 1u) / npi) < gridDim.x) npi = (npi + 1u) >> 1;
+    return npi;
 }
 
 // Invalid plan or permutation: every tile slot writes zeros (the wide units' rows included,
@@ -447,7 +459,7 @@ __device__ void zero_tile_slots(const RoutedGemm& g, uint32_t n_ntiles, uint32_t
 // the workgroup's column tiles, instead of being re-read from L2 for each of them.
 template <class Frag, int MODE, int NF, bool RESIDENT, bool DYNAMIC>
 __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, NF>& sm, const uint32_t* s_pref,
-                                           uint32_t n_ntiles, uint32_t npi, uint32_t n_chunks, const int32_t* s_grp) {
+                                           uint32_t n_ntiles, uint32_t npi_launch, const int32_t* s_grp) {
     constexpr bool dynamic = DYNAMIC;
     using S = Staged<MODE, NF>;
     using WC = WeightCopy<Frag, MODE, NF>;
@@ -456,6 +468,7 @@ __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, N
     auto& sa = sm.sa;
     auto& sw = sm.sw;
     uint32_t* s_dst = sm.s_dst;
+    const uint32_t npi = split_npi(s_pref[512], n_ntiles, npi_launch), n_chunks = (n_ntiles + npi - 1u) / npi;
     const uint32_t items = s_pref[512] * n_chunks;
     const uint32_t per = (items + 7u) >> 3, x = blockIdx.x & 7u, P = gridDim.x >> 3;
     const uint32_t i_end = (x + 1u) * per < items ? (x + 1u) * per : items;
@@ -693,7 +706,7 @@ __global__ __launch_bounds__(kV2Threads) void routed_gemm_staged_kernel(RoutedGe
         zero_tile_slots<MODE, NF>(g, n_ntiles, npi, n_chunks);
         return;
     }
-    tile_items<Frag, MODE, NF, RESIDENT, false>(g, sm, s_pref, n_ntiles, npi, n_chunks, s_grp);
+    tile_items<Frag, MODE, NF, RESIDENT, false>(g, sm, s_pref, n_ntiles, npi, s_grp);
 }
 
 

@@ -607,12 +607,12 @@ __global__ __launch_bounds__(kWideThreads) void routed_stage_kernel(RoutedGemm g
             wide_items<Prod, MODE, false>(g, nullptr, nullptr, n_ct, U, s_pref_w, sm.w.s_a, sm.w.s_b, sm.w.s_dst, nullptr,
                                           s_grp);
             __syncthreads();  // the wide phase's LDS is free
-            tile_items<Frag, MODE, 2, RESIDENT, true>(g, sm.t, s_pref_t, n_ntiles, npi, n_chunks, s_grp);
+            tile_items<Frag, MODE, 2, RESIDENT, true>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
         } else {
-            tile_items<Frag, MODE, 2, RESIDENT, false>(g, sm.t, s_pref_t, n_ntiles, npi, n_chunks, s_grp);
+            tile_items<Frag, MODE, 2, RESIDENT, false>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
         }
     } else {
-        tile_items<Frag, MODE, 2, RESIDENT, false>(g, sm.t, s_pref_t, n_ntiles, npi, n_chunks, s_grp);
+        tile_items<Frag, MODE, 2, RESIDENT, false>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
         if (U > 0u) {
             __syncthreads();  // the tile phase's LDS is free
             // Workgroups leave the tile phase at different times: the wide items are drawn.
@@ -659,7 +659,7 @@ template <class Prod, class Frag, int MODE>
 hipError_t launch_stage_t(const RoutedGemm& g, hipStream_t s) {
     const uint32_t n_ct = MODE == kGateUp ? g.n_out / 128u : g.n_out / 256u;
     const TilePlan tp = tile_plan<MODE, 2>(g.k, g.n_out);
-    const uint32_t blocks = wide_blocks(uint64_t(g.tile_capacity) * tp.n_chunks);
+    const uint32_t blocks = wide_blocks(uint64_t(g.tile_capacity) * tp.n_ntiles);
     if (tp.resident)
         routed_stage_kernel<Prod, Frag, MODE, true><<<blocks, kWideThreads, 0, s>>>(g, n_ct, tp.n_ntiles, tp.npi,
                                                                                    tp.n_chunks);
