@@ -256,6 +256,40 @@ struct FragQ80 {
     }
 };
 
+// Q8_0, the last 128 values of a row: group g owns block g (34 B). Nine dwords from the
+// 4-aligned offset 68 (g / 2) + 32 (g % 2) hold it, ending where the block pair ends (a row of
+// 128 values is 136 bytes): d in the low half of the first and the codes from byte 2 for an even
+// block, d in its high half and the codes from byte 4 for an odd one.
+struct HalfFragQ80 {
+    uint32_t w[9];
+    bool odd;
+    __device__ __forceinline__ void load(const uint8_t* blocks, int g) {
+        const uint8_t* p = blocks + 68 * (g >> 1) + 32 * (g & 1);
+        odd = (g & 1) != 0;
+#pragma unroll
+        for (int i = 0; i < 2; ++i) {
+            const u32x4 v = ld_global<u32x4>(p + 16 * i);
+#pragma unroll
+            for (int j = 0; j < 4; ++j) w[4 * i + j] = v[j];
+        }
+        w[8] = ld_global<uint32_t>(p + 32);
+    }
+    uint32_t q[8];
+    half2v dd;
+    __device__ __forceinline__ void prepare() {
+#pragma unroll
+        for (int i = 0; i < 8; ++i) q[i] = odd ? w[i + 1] : __builtin_amdgcn_alignbyte(w[i + 1], w[i], 2);
+        const _Float16 d = bits_f16(uint16_t(odd ? w[0] >> 16 : w[0] & 0xffffu));
+        dd = half2v{d, d};
+    }
+    __device__ __forceinline__ half8 step(int s) const {
+        const uint32_t x0 = q[2 * s] ^ 0x80808080u, x1 = q[2 * s + 1] ^ 0x80808080u;
+        const half2v p0 = q80_pair(x0, 0x04010400u, dd), p1 = q80_pair(x0, 0x04030402u, dd);
+        const half2v p2 = q80_pair(x1, 0x04010400u, dd), p3 = q80_pair(x1, 0x04030402u, dd);
+        return half8{p0[0], p0[1], p1[0], p1[1], p2[0], p2[1], p3[0], p3[1]};
+    }
+};
+
 // Q2_K (84 B / 256): scales[16] (low nibble scale, high nibble min), q[64] (2-bit codes,
 // four planes per byte), f16 d, f16 dmin. Value e = 128n + 32j + w uses bits 2j of
 // q[32n + w] and scale byte 8n + 2j + (w >= 16) (ggml's dequantize_row_q2_K). Group g

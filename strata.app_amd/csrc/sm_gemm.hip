@@ -320,18 +320,21 @@ hipError_t launch_staged(const RoutedGemm& g, hipStream_t s) {
     const uint32_t cap = device_cus() & ~7u;
     if (blocks > cap) blocks = cap;
     if (blocks < 8u) blocks = 8u;
-    if (p.resident)
-        routed_gemm_staged_kernel<Frag, MODE, NF, true><<<blocks, kV2Threads, 0, s>>>(g, p.n_ntiles, p.npi, p.n_chunks);
-    else
-        routed_gemm_staged_kernel<Frag, MODE, NF, false><<<blocks, kV2Threads, 0, s>>>(g, p.n_ntiles, p.npi, p.n_chunks);
-    return hipGetLastError();
+    auto go = [&](auto kern) {
+        kern<<<blocks, kV2Threads, 0, s>>>(g, p.n_ntiles, p.npi, p.n_chunks);
+        return hipGetLastError();
+    };
+    if constexpr (DirectWeights<Frag, MODE, true>::value)
+        if (g.k % kSlab != 0) return go(routed_gemm_staged_kernel<Frag, MODE, NF, true, true>);
+    return p.resident ? go(routed_gemm_staged_kernel<Frag, MODE, NF, true, false>)
+                      : go(routed_gemm_staged_kernel<Frag, MODE, NF, false, false>);
 }
 
 template <class Frag, int MODE>
 hipError_t launch_tiles(const RoutedGemm& g, hipStream_t s) {
     // Two fragments per wave: four (twice the multiplies per activation slab) measured no
     // faster on gfx950 and needs more than 256 VGPRs for Q4_K/Q2_K.
-    if (g.k % kSlab == 0 && g.n_out % Staged<MODE, 2>::kOut == 0) return launch_staged<Frag, MODE, 2>(g, s);
+    if (staged_fits<Frag, MODE, 2>(g.k, g.n_out)) return launch_staged<Frag, MODE, 2>(g, s);
     const uint32_t n_ntiles = MODE == kGateUp ? g.n_out / 64u : g.n_out / 128u;
     const uint32_t total = g.tile_capacity * n_ntiles;
     const uint32_t blocks = (total + 7u) & ~7u;
@@ -346,7 +349,7 @@ hipError_t launch_tiles(const RoutedGemm& g, hipStream_t s) {
 template <class Frag, int MODE>
 hipError_t launch_routed(Fmt fmt, const RoutedGemm& g, hipStream_t s) {
     if (g.wide_min == ~0u) return launch_tiles<Frag, MODE>(g, s);
-    if (g.k % kSlab == 0 && g.n_out % Staged<MODE, 2>::kOut == 0) return launch_stage(fmt, MODE == kGateUp, g, s);
+    if (staged_fits<Frag, MODE, 2>(g.k, g.n_out)) return launch_stage(fmt, MODE == kGateUp, g, s);
     const hipError_t e = launch_wide(fmt, MODE == kGateUp, g, s);
     return e != hipSuccess ? e : launch_tiles<Frag, MODE>(g, s);
 }

@@ -43,6 +43,16 @@ __device__ __forceinline__ uint32_t a_pos(uint32_t r, uint32_t c) {
     return 16u * (32u * (r >> 4) + 8u * (c >> 3) + (n & 7u)) + (n ^ (c & 7u));
 }
 
+// The 128 values past the last whole slab of a Q8_0 row (K % 256 == 128: the reference model's
+// K = 640) make a half slab of 64 x 128 values: lane group gq takes one 32-value block (four
+// k-steps, chunks 4 gq + s), so no lane multiplies padding. Its positions are grouped as
+// [rb][gq][n & 3][16]: a read's bank group is n ^ s as in a whole slab, and each 16-chunk group
+// holds the four chunks of the four rows n with the same n & 3.
+__device__ __forceinline__ uint32_t a_pos_half(uint32_t r, uint32_t c) {
+    const uint32_t n = r & 15u;
+    return 16u * (16u * (r >> 4) + 4u * (c >> 2) + (n & 3u)) + (n ^ (c & 3u));
+}
+
 template <int MODE>
 __device__ void zero_cols(const RoutedGemm& g, uint32_t r0, uint32_t r1, uint32_t c0, uint32_t c1, bool by_dst) {
     const uint32_t width = c1 - c0;
@@ -206,6 +216,24 @@ __device__ __forceinline__ void issue_slab(const _Float16* const (&asrc)[4], uin
     for (int j = 0; j < 4; ++j) issue_slab_part(asrc, k0, slab, wave, j);
 }
 
+// Copies the half slab at k0 (a_pos_half's inverse: position 16 Q + rho holds row
+// 16 (Q >> 4) + ((rho & 12) | (Q & 3)), chunk 4 ((Q >> 2) & 3) + ((rho & 3) ^ (Q & 3))); wave
+// instruction 2 wave + j reads 64 bytes of 16 rows.
+__device__ __forceinline__ void issue_half_slab(const RoutedGemm& g, const TileWork& t, uint32_t k0, _Float16* slab,
+                                                int wave, int lane) {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+        const uint32_t Q = 4u * (2u * wave + j) + (uint32_t(lane) >> 4), rho = uint32_t(lane) & 15u;
+        uint32_t row = t.a0 + 16u * (Q >> 4) + ((rho & 12u) | (Q & 3u));
+        if (row > t.a1 - 1u) row = t.a1 - 1u;
+        const _Float16* src = g.a + uint64_t(row) * g.k + k0 + 8u * (4u * ((Q >> 2) & 3u) + ((rho & 3u) ^ (Q & 3u)));
+        __builtin_amdgcn_global_load_lds(
+            reinterpret_cast<const __attribute__((address_space(1))) void*>(reinterpret_cast<uintptr_t>(src)),
+            reinterpret_cast<__attribute__((address_space(3))) void*>(reinterpret_cast<uintptr_t>(slab + (2 * wave + j) * 512)),
+            16, 0, 0);
+    }
+}
+
 // Geometry of a staged step with NF fragments per wave.
 template <int MODE, int NF>
 struct Staged {
@@ -253,6 +281,26 @@ __device__ __forceinline__ void slab_mma(const _Float16* buf, int n, int gq, con
 #pragma unroll
             for (int f = 0; f < NF; ++f) acc[f][rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[z][rb], b[z][f], acc[f][rb], 0, 0, 0);
         after_s(s);
+    }
+}
+
+// The half slab's four k-steps, as slab_mma.
+template <int RB>
+__device__ __forceinline__ void half_slab_mma(const _Float16* buf, int n, int gq, const HalfFragQ80& c, float4v (&acc)[1][4]) {
+    half8 a[2][RB], b[2];
+    auto fetch = [&](int s, int z) {
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb)
+            a[z][rb] = *reinterpret_cast<const half8*>(buf + 8u * a_pos_half(16u * rb + n, 4u * gq + s));
+        b[z] = c.step(s);
+    };
+    fetch(0, 0);
+#pragma unroll
+    for (int s = 0; s < 4; ++s) {
+        const int z = s & 1;
+        if (s + 1 < 4) fetch(s + 1, z ^ 1);
+#pragma unroll
+        for (int rb = 0; rb < RB; ++rb) acc[0][rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[z][rb], b[z], acc[0][rb], 0, 0, 0);
     }
 }
 
@@ -385,11 +433,13 @@ struct StagedBuffers {
     static_assert(65536u + kImage <= 143360u, "weight image too large for LDS");
 };
 
-// LDS of the staged tile kernels: the activation slabs (or the resident tile), the weight
-// image(s), the tile's destination rows (down) and the next dynamically drawn item.
-template <class Frag, int NF>
+// LDS of the staged tile kernels: the activation slabs (or the resident tile, with HALF its
+// half slab), the weight image(s), the tile's destination rows (down) and the next dynamically
+// drawn item.
+template <class Frag, int NF, bool HALF = false>
 struct TileSmem {
     _Float16 sa[2][64 * kSlab] __attribute__((aligned(1024)));
+    _Float16 sh[HALF ? 64 * kSlab / 2 : 8] __attribute__((aligned(1024)));
     uint8_t sw[StagedBuffers<Frag, NF>::kWBuf][StagedBuffers<Frag, NF>::kImage] __attribute__((aligned(1024)));
     uint32_t s_dst[64];  // down: destination row of each tile row
     uint32_t s_next;
@@ -417,7 +467,7 @@ template <int MODE, int NF>
 inline TilePlan tile_plan(uint32_t k, uint32_t n_out) {
     TilePlan p;
     p.n_ntiles = n_out / Staged<MODE, NF>::kOut;
-    const uint32_t n_slabs = k / kSlab;
+    const uint32_t n_slabs = k / kSlab;  // whole slabs; a half slab follows where K % 256 == 128
     p.npi = n_slabs <= 2 ? p.n_ntiles : (n_slabs >= 8 ? 1u : 8u / n_slabs);
     if (p.npi > p.n_ntiles) p.npi = p.n_ntiles;
     p.n_chunks = (p.n_ntiles + p.npi - 1) / p.npi;
@@ -434,6 +484,20 @@ inline TilePlan tile_plan(uint32_t k, uint32_t n_out) {
 __device__ __forceinline__ uint32_t split_npi(uint32_t tiles, uint32_t n_ntiles, uint32_t npi) {
     while (npi > 1u && tiles * ((n_ntiles + npi - 1u) / npi) < gridDim.x) npi = (npi + 1u) >> 1;
     return npi;
+}
+
+// Whether the staged tile kernels take a stage: whole column tiles, and K whole slabs or, for
+// the direct form (Q8_0 down), at most two whole slabs and a half one: three whole activation
+// slabs would not fit beside the output staging. At K = 640 (512 experts of 2560 columns, 20 rows
+// each: 891 MB of weights) the direct form takes 219 us per stage, 4.1 TB/s, where the plain tile
+// kernel took 301 us. Reductions that end elsewhere in a slab stay on the plain kernel.
+template <class Frag, int MODE>
+inline bool half_slab_fits(uint32_t k) {
+    return MODE == kDown && DirectWeights<Frag, MODE, true>::value && k % kSlab == kSlab / 2 && k / kSlab <= 2u;
+}
+template <class Frag, int MODE, int NF>
+inline bool staged_fits(uint32_t k, uint32_t n_out) {
+    return n_out % Staged<MODE, NF>::kOut == 0 && (k % kSlab == 0 || half_slab_fits<Frag, MODE>(k));
 }
 
 // Invalid plan or permutation: every tile slot writes zeros (the wide units' rows included,
@@ -457,8 +521,9 @@ __device__ void zero_tile_slots(const RoutedGemm& g, uint32_t n_ntiles, uint32_t
 // end, so the atomic's round trip overlaps the item's first copies.
 // RESIDENT (K <= 512): both activation slabs are copied once and stay in LDS for all of
 // the workgroup's column tiles, instead of being re-read from L2 for each of them.
-template <class Frag, int MODE, int NF, bool RESIDENT, bool DYNAMIC>
-__device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, NF>& sm, const uint32_t* s_pref,
+// HALF (direct form): K ends with a half slab, resident as well.
+template <class Frag, int MODE, int NF, bool RESIDENT, bool DYNAMIC, bool HALF = false>
+__device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, NF, HALF>& sm, const uint32_t* s_pref,
                                            uint32_t n_ntiles, uint32_t npi_launch, const int32_t* s_grp) {
     constexpr bool dynamic = DYNAMIC;
     using S = Staged<MODE, NF>;
@@ -528,6 +593,8 @@ __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, N
     if (RESIDENT)
         for (uint32_t sb = 0; sb < n_slabs; ++sb) issue_slab(asrc, sb * kSlab, sa[sb], wave);
     constexpr bool DIRECT = DirectWeights<Frag, MODE, RESIDENT>::value;
+    static_assert(!HALF || DIRECT, "the half slab belongs to the direct form");
+    if (HALF) issue_half_slab(g, t, n_slabs * kSlab, sm.sh, wave, lane);
     if constexpr (DIRECT) {
         // Steps are (column tile, half f): the wave's 16 weight rows of fragment f, rows
         // 128 f + 16 wave + n of the column tile, with every slab of them loaded at once, so a
@@ -536,11 +603,13 @@ __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, N
         // lines), are then fetched by one step, where loads a step apart fetched some of them
         // twice (lines evicted in between). The column tile's F32 results go out through LDS
         // (the weight image is unused here), so `parts` rows are written as whole 1 KB pieces.
-        auto load_step = [&](auto& c, uint32_t tile, int f) {
+        auto load_step = [&](auto& c, HalfFragQ80& h, auto ns_const, uint32_t tile, int f) {
+            constexpr int NS = decltype(ns_const)::value;
             const uint32_t r = (t.nt_begin + tile) * S::kImageRows + 128u * uint32_t(f) + 16u * uint32_t(wave) + uint32_t(n);
+            const uint8_t* row = t.w0 + uint64_t(r) * g.row_bytes;
 #pragma unroll
-            for (int sb = 0; sb < int(sizeof(c) / sizeof(c[0])); ++sb)
-                c[sb][0].template load<FromGlobal>(t.w0 + uint64_t(r) * g.row_bytes + uint64_t(sb) * SB, gq);
+            for (int sb = 0; sb < NS; ++sb) c[sb][0].template load<FromGlobal>(row + uint64_t(sb) * SB, gq);
+            if constexpr (HALF) h.load(row + uint64_t(NS) * SB, gq);
         };
         // The finished column tile: accumulators -> LDS [row][256 + 4 pad] (the pad puts the
         // four lane groups' rows in distinct banks), then each wave stores 8 rows, 64 lanes x 16
@@ -580,41 +649,47 @@ __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, N
         };
         auto run_direct = [&](auto rb_const, auto ns_const) {
             constexpr int RB = decltype(rb_const)::value;
-            constexpr int NS = decltype(ns_const)::value;  // slabs (K = 256 NS)
+            constexpr int NS = decltype(ns_const)::value;  // whole slabs (K = 256 NS, or + 128 with HALF)
             float4v acc[2][1][4];
 #pragma unroll
             for (int f = 0; f < 2; ++f)
 #pragma unroll
                 for (int rb = 0; rb < 4; ++rb) acc[f][0][rb] = float4v{0, 0, 0, 0};
             const uint32_t n_tiles = t.nt_end - t.nt_begin;
-            Frag fa[NS][1], fb[NS][1];
-            load_step(fa, 0, 0);
-            auto do_step = [&](Frag (&cur)[NS][1], float4v (&acc_f)[1][4]) {
+            Frag fa[NS > 0 ? NS : 1][1], fb[NS > 0 ? NS : 1][1];
+            HalfFragQ80 ha, hb;
+            load_step(fa, ha, ns_const, 0, 0);
+            auto do_step = [&](auto& cur, HalfFragQ80& h, float4v (&acc_f)[1][4]) {
 #pragma unroll
                 for (int sb = 0; sb < NS; ++sb) {
                     cur[sb][0].prepare();
                     slab_mma<Frag, 1, RB>(sa[sb], n, gq, cur[sb], acc_f, [](int) {});
                 }
+                if constexpr (HALF) {
+                    h.prepare();
+                    half_slab_mma<RB>(sm.sh, n, gq, h, acc_f);
+                }
             };
             for (uint32_t tile = 0; tile < n_tiles; ++tile) {
                 __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // fa: (tile, f = 0)
                 if (tile == 0) __syncthreads();                         // the resident slabs
-                load_step(fb, tile, 1);
+                load_step(fb, hb, ns_const, tile, 1);
                 // The loads stay ahead of this step's work (left alone, the scheduler sinks them
                 // below the multiplies, and the next step then waits for their whole latency).
                 __builtin_amdgcn_sched_barrier(0);
-                do_step(fa, acc[0]);
+                do_step(fa, ha, acc[0]);
                 __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // fb: (tile, f = 1)
-                load_step(fa, tile + 1 < n_tiles ? tile + 1 : tile, 0);
+                load_step(fa, ha, ns_const, tile + 1 < n_tiles ? tile + 1 : tile, 0);
                 __builtin_amdgcn_sched_barrier(0);
-                do_step(fb, acc[1]);
+                do_step(fb, hb, acc[1]);
                 epilogue(rb_const, acc, tile);
             }
             __asm__ volatile("s_waitcnt vmcnt(0)" ::: "memory");  // the repeated last loads
         };
         auto run_ns = [&](auto rb_const) {
             if (n_slabs == 2u) run_direct(rb_const, std::integral_constant<int, 2>());
-            else run_direct(rb_const, std::integral_constant<int, 1>());
+            else if (!HALF || n_slabs == 1u) run_direct(rb_const, std::integral_constant<int, 1>());
+            else if constexpr (HALF) run_direct(rb_const, std::integral_constant<int, 0>());
         };
         switch ((t.a1 - t.a0 + 15u) / 16u) {  // workgroup-uniform
             case 1: run_ns(std::integral_constant<int, 1>()); break;
@@ -695,10 +770,10 @@ __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, N
     }
 }
 
-template <class Frag, int MODE, int NF, bool RESIDENT>
+template <class Frag, int MODE, int NF, bool RESIDENT, bool HALF>
 __global__ __launch_bounds__(kV2Threads) void routed_gemm_staged_kernel(RoutedGemm g, uint32_t n_ntiles, uint32_t npi,
                                                                         uint32_t n_chunks) {
-    __shared__ TileSmem<Frag, NF> sm;
+    __shared__ TileSmem<Frag, NF, HALF> sm;
     __shared__ uint32_t s_pref[513], s_wsum[8], s_flag;
     __shared__ int32_t s_grp[kGrpWords];
     const uint32_t flag = scan_small_tiles(g, s_pref, s_wsum, &s_flag, s_grp);
@@ -706,7 +781,7 @@ __global__ __launch_bounds__(kV2Threads) void routed_gemm_staged_kernel(RoutedGe
         zero_tile_slots<MODE, NF>(g, n_ntiles, npi, n_chunks);
         return;
     }
-    tile_items<Frag, MODE, NF, RESIDENT, false>(g, sm, s_pref, n_ntiles, npi, s_grp);
+    tile_items<Frag, MODE, NF, RESIDENT, false, HALF>(g, sm, s_pref, n_ntiles, npi, s_grp);
 }
 
 

@@ -584,13 +584,13 @@ __global__ __launch_bounds__(kWideThreads) void wide_gemm_kernel(RoutedGemm g, c
 // streams its expert's whole weight matrix through L2, which would evict the activation rows
 // that concurrently running wide units share across column tiles; taken first, the tiles
 // overlap the wide units only at the boundary.
-template <class Prod, class Frag, int MODE, bool RESIDENT>
+template <class Prod, class Frag, int MODE, bool RESIDENT, bool HALF>
 __global__ __launch_bounds__(kWideThreads) void routed_stage_kernel(RoutedGemm g, uint32_t n_ct, uint32_t n_ntiles,
                                                                     uint32_t npi, uint32_t n_chunks) {
     static_assert(kWideThreads == kV2Threads, "one workgroup shape for both phases");
     __shared__ union Smem {
         WideSmem w;
-        TileSmem<Frag, 2> t;
+        TileSmem<Frag, 2, HALF> t;
     } sm;
     __shared__ uint32_t s_pref_w[513], s_pref_t[513], s_wsum[8], s_tsum[8], s_flag, s_next_w;
     __shared__ int32_t s_grp[kGrpWords];
@@ -607,12 +607,12 @@ __global__ __launch_bounds__(kWideThreads) void routed_stage_kernel(RoutedGemm g
             wide_items<Prod, MODE, false>(g, nullptr, nullptr, n_ct, U, s_pref_w, sm.w.s_a, sm.w.s_b, sm.w.s_dst, nullptr,
                                           s_grp);
             __syncthreads();  // the wide phase's LDS is free
-            tile_items<Frag, MODE, 2, RESIDENT, true>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
+            tile_items<Frag, MODE, 2, RESIDENT, true, HALF>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
         } else {
-            tile_items<Frag, MODE, 2, RESIDENT, false>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
+            tile_items<Frag, MODE, 2, RESIDENT, false, HALF>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
         }
     } else {
-        tile_items<Frag, MODE, 2, RESIDENT, false>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
+        tile_items<Frag, MODE, 2, RESIDENT, false, HALF>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
         if (U > 0u) {
             __syncthreads();  // the tile phase's LDS is free
             // Workgroups leave the tile phase at different times: the wide items are drawn.
@@ -660,13 +660,14 @@ hipError_t launch_stage_t(const RoutedGemm& g, hipStream_t s) {
     const uint32_t n_ct = MODE == kGateUp ? g.n_out / 128u : g.n_out / 256u;
     const TilePlan tp = tile_plan<MODE, 2>(g.k, g.n_out);
     const uint32_t blocks = wide_blocks(uint64_t(g.tile_capacity) * tp.n_ntiles);
-    if (tp.resident)
-        routed_stage_kernel<Prod, Frag, MODE, true><<<blocks, kWideThreads, 0, s>>>(g, n_ct, tp.n_ntiles, tp.npi,
-                                                                                   tp.n_chunks);
-    else
-        routed_stage_kernel<Prod, Frag, MODE, false><<<blocks, kWideThreads, 0, s>>>(g, n_ct, tp.n_ntiles, tp.npi,
-                                                                                    tp.n_chunks);
-    return hipGetLastError();
+    auto go = [&](auto kern) {
+        kern<<<blocks, kWideThreads, 0, s>>>(g, n_ct, tp.n_ntiles, tp.npi, tp.n_chunks);
+        return hipGetLastError();
+    };
+    if constexpr (DirectWeights<Frag, MODE, true>::value)
+        if (g.k % kSlab != 0) return go(routed_stage_kernel<Prod, Frag, MODE, true, true>);
+    return tp.resident ? go(routed_stage_kernel<Prod, Frag, MODE, true, false>)
+                       : go(routed_stage_kernel<Prod, Frag, MODE, false, false>);
 }
 
 template <class Prod, int MODE>

@@ -3,8 +3,7 @@
 Every group here is below 128 entries, so both expert stages run on the tile kernels; the
 shapes cover Q4_K, Q2_K and Q8_0 weights on both stages, reductions of one to five
 256-value slabs (activation slabs resident or streamed), one to eight column tiles per work
-item, a down reduction of 384 values, which runs on the plain tile kernel, and more gate/up
-items than workgroups (items run back to back). Each case checks every token of both stages and
+item, a down reduction of 384 values, which ends with half a slab, and more gate/up items than workgroups (items run back to back), and few row tiles split over the workgroups. Each case checks every token of both stages and
 the layer against the CPU oracle with the benchmark configurations' bars (gate/up within
 1 F16 ulp, down parts within 2e-5 + 2e-5 |x|, layer max-abs 2e-2 and rel-L2 5e-3), and the failure
 paths (a missing expert address zeroes that group's rows, leaves every other row as the clean
@@ -30,7 +29,7 @@ def _cases(layer, moe):
         "q2k_q80": C("tiles_q80", 256, 1024, 16, 4, 1024, 0, moe.Q2_K, moe.Q8_0, moe.F16, seed=302),
         # gate/up Q4_K: 1 slab, 4 column tiles of 128; down Q8_0: 2 slabs, 1 column tile
         "q80_2slab": C("tiles_q80b", 128, 256, 8, 2, 512, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=303),
-        # gate/up Q4_K: 3 column tiles; down K = 384 on the plain tile kernel
+        # gate/up Q4_K: 3 column tiles; down K = 384: one whole slab and a half one
         "odd_tiles": C("tiles_odd", 192, 512, 12, 2, 384, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=304),
         # 512 gate/up items (128 groups x 4 column tiles) on at most 256 workgroups: each
         # workgroup runs items back to back, the next one's copies issued by the current one
@@ -130,3 +129,14 @@ def test_short_reduction_rows(moe, layer, orc, gpu_ctx, stream, ff):
     print(f"case tiles short reduction {ff}", flush=True)
     cfg = layer.LayerConfig("tiles_short", 96, 256, 12, 2, ff, 0, moe.Q8_0, moe.Q8_0, moe.F16, seed=311)
     _check_layer(moe, layer, orc, gpu_ctx, stream, cfg)
+
+
+@pytest.mark.parametrize("rows,ff,zipf", [(33, 640, 0.0), (512, 640, 1.1), (512, 384, 1.1), (512, 128, 1.1)])
+def test_half_slab_reduction(moe, layer, orc, gpu_ctx, stream, rows, ff, zipf):
+    """Down reductions of 0, 1 and 2 whole slabs and a half one, on tiles alone and (skewed) beside
+    wide units."""
+    print(f"case tiles half slab K {ff} rows {rows}", flush=True)
+    cfg = layer.LayerConfig("tiles_half", rows, 768, 32, 4, ff, 0, moe.Q4_K, moe.Q8_0, moe.F16, zipf_s=zipf, seed=312)
+    ws = _check_layer(moe, layer, orc, gpu_ctx, stream, cfg)
+    counts = np.bincount(gu.host(ws.ids, np.int32), minlength=cfg.n_experts)
+    assert (counts.max() >= 128) == (zipf > 0)
