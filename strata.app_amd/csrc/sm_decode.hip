@@ -9,6 +9,7 @@
 // 32-value Q8_1 blocks of K, and every lane keeps one accumulator per entry of the group.
 // Integer block dots run on v_dot4_i32_i8 (codes times Q8_1 codes, exact), then the block's
 // float scales; a butterfly over the row's lanes finishes the row.
+#include <stddef.h>
 #include <stdint.h>
 
 #include "sm_device.h"
@@ -256,24 +257,21 @@ __device__ __forceinline__ int sdot4(uint32_t a, uint32_t b, int c) {
     return __builtin_amdgcn_sdot4(int(a), int(b), c, false);
 }
 
-// A Q8_1 block of an activation row: its 8 code words and the float d.
+// A Q8_1 block of an activation row: its 8 code words, the float d, and the sums of the first
+// and the last 16 codes (the min terms' factors: they depend on the activation alone, so the
+// workgroup takes them once when it stages the block, not once per weight row).
 struct Act {
     uint32_t q[8];
     float d;
+    int t0, t1;
 };
-__device__ __forceinline__ Act load_act(const uint8_t* blk) {  // 36-byte blocks: 4-byte aligned
-    Act a;
-#pragma unroll
-    for (int i = 0; i < 8; ++i) a.q[i] = ld_global<uint32_t>(blk + 4 + 4 * i);
-    a.d = f16_lo(ld_global<uint32_t>(blk));
-    return a;
-}
 
 // Weight side of a row, per format, in units that a lane takes whole: a Q4_K or Q2_K
 // super-block (256 values) or a pair of Q8_0 blocks (64 values). raw() issues the unit's
 // loads (kRaw dwords, every byte of the unit, nothing else); dot() takes sub-block s (32
 // values) of the loaded unit against one activation block.
 typedef uint32_t u32x4a __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 struct UnitQ80 {  // 2 x 34 B: d0, q0[32], d1, q1[32]; 4-byte aligned (rows hold whole pairs)
     static constexpr uint32_t kVals = 64, kSub = 2, kRaw = 17;
@@ -328,13 +326,10 @@ struct UnitQ4K {  // 144 B: d, dmin, scales[12], qs[128]; 16-byte aligned
             sc = int((byte(j + 4) & 0xFu) | ((byte(j - 4) >> 6) << 4));
             mn = int((byte(j + 4) >> 4) | ((byte(j) >> 6) << 4));
         }
-        int s = 0, t = 0;
+        int s = 0;
 #pragma unroll
-        for (int i = 0; i < 8; ++i) {
-            s = sdot4((r[q0 + i] >> sh) & 0x0F0F0F0Fu, x.q[i], s);
-            t = sdot4(0x01010101u, x.q[i], t);
-        }
-        const float sd = x.d * float(s * sc), sm = x.d * float(t * mn);
+        for (int i = 0; i < 8; ++i) s = sdot4((r[q0 + i] >> sh) & 0x0F0F0F0Fu, x.q[i], s);
+        const float sd = x.d * float(s * sc), sm = x.d * float((x.t0 + x.t1) * mn);
         return acc + __builtin_fmaf(-f16_hi(r[0]), sm, f16_lo(r[0]) * sd);  // q4_K: fma(-dm.y, sm, dm.x * sd), then acc + v
     }
 };
@@ -356,16 +351,14 @@ struct UnitQ2K {  // 84 B: scales[16] @0, q[64] @16, d @80, dmin @82; 4-byte ali
         const uint32_t nn = bb >> 2, j = bb & 3u;
         const uint32_t scw = r[2 * nn + (j >> 1)];
         const uint32_t s0 = (scw >> (16u * (j & 1u))) & 0xffu, s1 = (scw >> (16u * (j & 1u) + 8u)) & 0xffu;
-        int a0 = 0, a1 = 0, t0 = 0, t1 = 0;
+        int a0 = 0, a1 = 0;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
             a0 = sdot4((r[4 + 8 * nn + i] >> (2u * j)) & 0x03030303u, x.q[i], a0);
-            t0 = sdot4(0x01010101u, x.q[i], t0);
             a1 = sdot4((r[4 + 8 * nn + 4 + i] >> (2u * j)) & 0x03030303u, x.q[4 + i], a1);
-            t1 = sdot4(0x01010101u, x.q[4 + i], t1);
         }
         const float sd = x.d * float(a0 * int(s0 & 0xFu) + a1 * int(s1 & 0xFu));
-        const float sm = x.d * float(t0 * int(s0 >> 4) + t1 * int(s1 >> 4));
+        const float sm = x.d * float(x.t0 * int(s0 >> 4) + x.t1 * int(s1 >> 4));
         return acc + __builtin_fmaf(-f16_hi(r[20]), sm, f16_lo(r[20]) * sd);
     }
 };
@@ -387,11 +380,23 @@ struct UnitQ2K {  // 84 B: scales[16] @0, q[64] @16, d @80, dmin @82; 4-byte ali
 
 __host__ __device__ constexpr uint32_t matvec_rows_per_block(uint32_t lpr) { return 4u * (64u / lpr); }
 
+// LDS of the staged activation units: a unit's kSub blocks of 8 code words and 4 words of pad,
+// then, past all units, {d, code sums} per block and 2 words of pad per unit. The lanes of a row
+// read the same block of consecutive units at once: without the pad a 256-value unit is 256 bytes,
+// all 64 banks, and every 16-byte read of the row's ten or sixteen lanes hit the same four banks.
+// With it they sit in distinct bank groups (launch times by events: gate/up at T = 8, Q4_K,
+// K = 2560 38.3 -> 33.7 us; at T = 4, Q2_K, K = 4096 62.4 -> 31.0 us, both with the code sums
+// staged instead of summed again for every weight row).
+template <class Unit> struct ActLds {
+    static constexpr uint32_t kCodes = Unit::kSub * 8u + 4u, kMeta = Unit::kSub * 2u + 2u;
+    static __host__ __device__ constexpr uint32_t words(uint32_t units) { return units * (kCodes + kMeta); }
+};
+
 template <class Unit, int MODE, uint32_t LPR>
 __global__ __launch_bounds__(256, 4) void moe_matvec_kernel(DecodeMatvec m) {  // >= 4 waves per SIMD
     constexpr uint32_t RPW = 64u / LPR, RPI = 4u * RPW;  // rows per wave, rows per slice
     constexpr bool kPow2 = (LPR & (LPR - 1u)) == 0u;
-    // LDS: codes [entry][block] (8 words), then d [entry][block], then results [slice row][entry]
+    // LDS: codes [entry][unit], then d and code sums [entry][unit] (ActLds), then results [slice row][entry]
     extern __shared__ uint32_t act_s[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t g = blockIdx.y;
@@ -399,9 +404,17 @@ __global__ __launch_bounds__(256, 4) void moe_matvec_kernel(DecodeMatvec m) {  /
     if (g >= 80u) return;
     // A plan whose header is unusable: workgroup (0, 0) reports it and zeroes every output row
     // this stage could have written.
-    // Every plan field this workgroup needs, read in one round trip (g < 80: all inside the plan).
-    const uint32_t p_entries = P->n_entries, p_groups = P->n_groups;
-    const int32_t p_s = P->grp_start[g], p_t = P->grp_start[g + 1], p_e = P->grp_e[g];
+    // Every plan field this workgroup needs, read in one round trip (g < 80: all inside the plan),
+    // one field per lane: loads of uniform addresses would each be waited for on their way into
+    // scalar registers, one round trip per field (twelve of them, eight for the entries below,
+    // made T = 1's gate/up 10.4 us by events instead of 8.9 and its down 9.9 instead of 8.2).
+    const uint32_t* pw = reinterpret_cast<const uint32_t*>(m.plan);
+    constexpr uint32_t kGrpE = offsetof(DecodePlan, grp_e) / 4u, kStart = offsetof(DecodePlan, grp_start) / 4u;
+    const uint32_t hdr = ld_global<uint32_t>(pw + (lane < 2u ? lane : lane < 4u ? kStart + g + (lane - 2u) : kGrpE + g));
+    auto field = [](uint32_t v, int l) { return uint32_t(__builtin_amdgcn_readlane(int(v), l)); };
+    const uint32_t p_groups = field(hdr, 0), p_entries = field(hdr, 1);
+    const int32_t p_s = int32_t(field(hdr, 2)), p_t = int32_t(field(hdr, 3)), p_e = int32_t(field(hdr, 4));
+    static_assert(offsetof(DecodePlan, n_groups) == 0 && offsetof(DecodePlan, n_entries) == 4, "header lanes 0 and 1");
     const bool plan_ok = p_entries == m.n_entries && p_groups <= m.n_entries;  // a group holds >= 1 entry
     if (!plan_ok) {
         if (g != 0u || blockIdx.x != 0u) return;
@@ -422,27 +435,29 @@ __global__ __launch_bounds__(256, 4) void moe_matvec_kernel(DecodeMatvec m) {  /
     const uint32_t a0 = uint32_t(p_s), a1 = uint32_t(p_t), ex = uint32_t(p_e);
     const uint32_t n_e = a1 - a0;
     // Entries: activation row (gate/up: the token; down: the grouped entry) and output row
-    // (gate/up: the grouped entry; down: the route index from ent_dst).
-    uint32_t arow[8], orow[8];
+    // (gate/up: the grouped entry; down: the route index from ent_dst). The looked-up row of each
+    // entry is a byte of `rows8` (tokens < 8, route indices < 80; 255: names no row), so that no
+    // indexed array of them lives in scratch.
+    // Entries (lanes 0-7) and the expert's addresses (lanes 8-13) are one more round trip.
+    constexpr uint32_t kEnt = (MODE == kGateUp ? offsetof(DecodePlan, ent_tok) : offsetof(DecodePlan, ent_dst)) / 4u;
+    const uint32_t* aw = reinterpret_cast<const uint32_t*>(m.addresses + 3u * ex);
+    const uint32_t* src = lane < 8u ? pw + kEnt + a0 + (lane < n_e ? lane : n_e - 1u)
+                                    : aw + (lane < 14u ? lane - 8u : 0u);
+    const uint32_t got = ld_global<uint32_t>(src);
+    uint64_t rows8 = 0;
     bool entries_ok = true;
 #pragma unroll
-    for (uint32_t c = 0; c < 8u; ++c) {
-        const uint32_t a = a0 + (c < n_e ? c : n_e - 1u);
-        if (MODE == kGateUp) {
-            const int32_t t = P->ent_tok[a];
-            entries_ok = entries_ok && t >= 0 && uint32_t(t) < m.act_rows;
-            arow[c] = uint32_t(t);
-            orow[c] = a;
-        } else {
-            const int32_t dd = P->ent_dst[a];
-            entries_ok = entries_ok && dd >= 0 && uint32_t(dd) < m.n_entries;
-            arow[c] = a;
-            orow[c] = uint32_t(dd);
-        }
+    for (int c = 0; c < 8; ++c) {
+        const uint32_t v = field(got, c);
+        const bool in = v < (MODE == kGateUp ? m.act_rows : m.n_entries);  // negative: not below either
+        entries_ok = entries_ok && in;
+        rows8 |= uint64_t(in ? v : 255u) << (8u * uint32_t(c));
     }
-    const uint64_t* addr = m.addresses + 3u * ex;
-    const uint8_t* w0 = reinterpret_cast<const uint8_t*>(MODE == kGateUp ? addr[0] : addr[2]);
-    const uint8_t* w1 = reinterpret_cast<const uint8_t*>(MODE == kGateUp ? addr[1] : addr[2]);
+    auto arow = [&](uint32_t c) { return MODE == kGateUp ? uint32_t(rows8 >> (8u * c)) & 255u : a0 + c; };
+    auto orow = [&](uint32_t c) { return MODE == kGateUp ? a0 + c : uint32_t(rows8 >> (8u * c)) & 255u; };
+    auto address = [&](int i) { return reinterpret_cast<const uint8_t*>(uint64_t(field(got, 8 + 2 * i)) | (uint64_t(field(got, 9 + 2 * i)) << 32)); };
+    const uint8_t* w0 = address(MODE == kGateUp ? 0 : 2);
+    const uint8_t* w1 = address(MODE == kGateUp ? 1 : 2);
     const uint32_t fault = entries_ok ? weight_fault(w0, w1) : 2u;
     const uint32_t n_rows = MODE == kGateUp ? 2u * m.out_width : m.out_width;
     const uint32_t rows_wg = m.iters * RPI, r_first = rows_wg * blockIdx.x;
@@ -453,7 +468,7 @@ __global__ __launch_bounds__(256, 4) void moe_matvec_kernel(DecodeMatvec m) {  /
             float* out = up ? m.out1 : m.out0;
             const uint32_t col = up ? i - m.out_width : i;
             for (uint32_t c = 0; c < n_e; ++c)  // a damaged entry's row cannot be named: skipped
-                if (orow[c] < m.n_entries) out[uint64_t(orow[c]) * m.out_width + col] = 0.0f;
+                if (orow(c) < m.n_entries) out[uint64_t(orow(c)) * m.out_width + col] = 0.0f;
         }
         if (tid == 0 && blockIdx.x == 0u) atomicOr(m.status, fault);
         return;
@@ -469,50 +484,46 @@ __global__ __launch_bounds__(256, 4) void moe_matvec_kernel(DecodeMatvec m) {  /
         const bool up = MODE == kGateUp && rowc >= m.out_width;
         return (up ? w1 : w0) + uint64_t(up ? rowc - m.out_width : rowc) * m.row_bytes;
     };
-    uint32_t* codes_s = act_s;                                               // [entry][block][8]
-    float* d_s = reinterpret_cast<float*>(act_s + m.max_group * nblk * 8u);  // [entry][block]
-    float* res_s = d_s + m.max_group * nblk;                                 // [slice row][entry]
-    // Stage the group's activation blocks (n_e rows of nblk Q8_1 blocks) into LDS. The first
-    // kStageRegs words per thread are loaded into registers before the first slice's weight
+    using L = ActLds<Unit>;
+    uint32_t* meta_s = act_s + m.max_group * nunit * L::kCodes;
+    float* res_s = reinterpret_cast<float*>(act_s + L::words(m.max_group * nunit));  // [slice row][entry]
+    // Stage the group's activation blocks (n_e rows of nblk Q8_1 blocks) into LDS, one block per
+    // thread. A thread's first block is loaded into registers before the first slice's weight
     // units are requested and stored after, so the two round trips overlap (the loads return in
-    // order, so storing the staged words waits only for them); the barrier then waits for the
-    // LDS stores alone and leaves the weight loads in flight.
-    constexpr uint32_t kStageRegs = 4;
-    const uint32_t n_words = n_e * nblk * 9u;  // >= 9
-    const uint32_t d_base = m.max_group * nblk * 8u;
-    auto stage_src = [&](uint32_t i) {
-        const uint32_t c = i / (nblk * 9u), rem = i - c * nblk * 9u, b = rem / 9u, w = rem - b * 9u;
-        return m.act + (uint64_t(arow[c]) * nblk + b) * kQ81Bytes + 4u * w;
+    // order, so storing the staged block waits only for it); the barrier then waits for the LDS
+    // stores alone and leaves the weight loads in flight.
+    const uint32_t n_blocks = n_e * nblk;  // >= 1
+    struct Staged {
+        u32x4a lo, hi;
+        uint32_t ds;
     };
-    // LDS word of staged word i: its block's d (as F32) or one of its 8 code words.
-    auto stage_dst = [&](uint32_t i, uint32_t& v) {
-        const uint32_t c = i / (nblk * 9u), rem = i - c * nblk * 9u, b = rem / 9u, w = rem - b * 9u;
-        v = w == 0u ? f32_bits(f16_lo(v)) : v;
-        return w == 0u ? d_base + c * nblk + b : (c * nblk + b) * 8u + (w - 1u);
+    auto stage_load = [&](uint32_t i) {
+        const uint32_t c = i / nblk;
+        const uint8_t* p = m.act + (uint64_t(arow(c)) * nblk + (i - c * nblk)) * kQ81Bytes;
+        return Staged{ld_global<u32x4a>(p + 4), ld_global<u32x4a>(p + 20), ld_global<uint32_t>(p)};
     };
-    // Branch-free, so the stores wait for the staged words only: loads clamped into the range,
-    // and a thread past it stores to the first result word, which the first slice overwrites.
-    uint32_t sv[kStageRegs];
+    auto stage_store = [&](uint32_t i, const Staged& v) {
+        const uint32_t unit = i / Unit::kSub, sb = i % Unit::kSub;  // nblk is a multiple of kSub
+        uint32_t* q = act_s + unit * L::kCodes + 8u * sb;
+        int t0 = 0, t1 = 0;
 #pragma unroll
-    for (uint32_t j = 0; j < kStageRegs; ++j) {
-        const uint32_t i = tid + 256u * j;
-        sv[j] = ld_global<uint32_t>(stage_src(i < n_words ? i : n_words - 1u));
-    }
+        for (int j = 0; j < 4; ++j) {
+            t0 = sdot4(0x01010101u, v.lo[j], t0);
+            t1 = sdot4(0x01010101u, v.hi[j], t1);
+        }
+        *reinterpret_cast<u32x4*>(q) = u32x4{v.lo[0], v.lo[1], v.lo[2], v.lo[3]};
+        *reinterpret_cast<u32x4*>(q + 4) = u32x4{v.hi[0], v.hi[1], v.hi[2], v.hi[3]};
+        u32x2* meta = reinterpret_cast<u32x2*>(meta_s + unit * L::kMeta + 2u * sb);
+        *meta = u32x2{f32_bits(f16_lo(v.ds)), (uint32_t(t0) & 0xffffu) | (uint32_t(t1) << 16)};
+    };
+    // Loads clamped into the range, so no branch sits between them and the weight loads.
+    const Staged first = stage_load(tid < n_blocks ? tid : n_blocks - 1u);
+    __asm__ volatile("" ::: "memory");  // the staging loads stay ahead of the weight loads
     uint32_t r[Unit::kRaw];
     Unit::raw(row_ptr(0u), u, r);
-#pragma unroll
-    for (uint32_t j = 0; j < kStageRegs; ++j) {
-        const uint32_t i = tid + 256u * j;
-        uint32_t v = sv[j];
-        const uint32_t at = stage_dst(i < n_words ? i : n_words - 1u, v);
-        act_s[i < n_words ? at : d_base + m.max_group * nblk] = v;
-    }
-    if (n_words > 256u * kStageRegs)  // more than eight entries' worth at d = 2560: the rest in the plain way
-        for (uint32_t i = tid + 256u * kStageRegs; i < n_words; i += 256u) {
-            uint32_t v = ld_global<uint32_t>(stage_src(i));
-            const uint32_t at = stage_dst(i, v);  // converts v first
-            act_s[at] = v;
-        }
+    __asm__ volatile("" ::: "memory");
+    if (tid < n_blocks) stage_store(tid, first);
+    for (uint32_t i = tid + 256u; i < n_blocks; i += 256u) stage_store(i, stage_load(i));
     __asm__ volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
     for (uint32_t it = 0; it < m.iters; ++it) {
         const uint32_t lr = it * RPI + wave * RPW + (lane_ok ? rin : 0u);
@@ -528,16 +539,18 @@ __global__ __launch_bounds__(256, 4) void moe_matvec_kernel(DecodeMatvec m) {  /
             if (unit_ok) {
 #pragma unroll
                 for (uint32_t sb = 0; sb < Unit::kSub; ++sb) {
-                    const uint32_t b = u * Unit::kSub + sb;
-                    const uint32_t* cs = codes_s + (c * nblk + b) * 8u;
+                    const uint32_t* cs = act_s + (c * nunit + u) * L::kCodes + 8u * sb;
                     const u32x4 qa = *reinterpret_cast<const u32x4*>(cs), qb = *reinterpret_cast<const u32x4*>(cs + 4);
+                    const u32x2 meta = *reinterpret_cast<const u32x2*>(meta_s + (c * nunit + u) * L::kMeta + 2u * sb);
                     Act a;
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
                         a.q[i] = qa[i];
                         a.q[4 + i] = qb[i];
                     }
-                    a.d = d_s[c * nblk + b];
+                    a.d = bits_f32(meta[0]);
+                    a.t0 = int(meta[1] << 16) >> 16;
+                    a.t1 = int(meta[1]) >> 16;
                     acc = Unit::dot(r, sb, a, acc);
                     // The next pair's LDS reads stay below this pair's dots (register budget).
                     if (sb & 1u) __builtin_amdgcn_sched_barrier(0);
@@ -565,7 +578,7 @@ __global__ __launch_bounds__(256, 4) void moe_matvec_kernel(DecodeMatvec m) {  /
         const bool up = MODE == kGateUp && row >= m.out_width;
         float* out = up ? m.out1 : m.out0;
         const uint32_t col = up ? row - m.out_width : row;
-        out[uint64_t(orow[c]) * m.out_width + col] = res_s[lr * m.max_group + c];
+        out[uint64_t(orow(c)) * m.out_width + col] = res_s[lr * m.max_group + c];
     }
 }
 
@@ -721,7 +734,6 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
                                 xv[(2u * j + 1u) % VPC] = f16_hi(q[j]);
                             }
                         } else {
-                            typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
                             const u32x2 q = *reinterpret_cast<const u32x2*>(xp);
                             xv[0] = f16_lo(q[0]);
                             xv[1] = f16_hi(q[0]);
@@ -904,7 +916,7 @@ template <class Unit, int MODE>
 hipError_t launch_matvec_t(const DecodeMatvec& mm, hipStream_t s) {
     DecodeMatvec m = mm;
     const uint32_t n_rows = MODE == kGateUp ? 2u * m.out_width : m.out_width;
-    const uint32_t nblk = m.k / 32u, nunit = m.k / Unit::kVals;
+    const uint32_t nunit = m.k / Unit::kVals;
     if (nunit == 0u || nunit > 64u || m.k % Unit::kVals != 0u) return hipErrorInvalidValue;  // host-checked
     if (m.max_group == 0u || m.max_group > 8u || m.n_entries == 0u || m.n_entries > 80u) return hipErrorInvalidValue;
     uint32_t lpr = 1;
@@ -919,7 +931,7 @@ hipError_t launch_matvec_t(const DecodeMatvec& mm, hipStream_t s) {
     m.iters = per_iter >= 4096u ? 4u : per_iter >= 2048u ? 2u : 1u;
     // One grid row per possible group: a valid plan has at most one group per entry (<= 80).
     const dim3 grid((slices + m.iters - 1u) / m.iters, m.n_entries);
-    const size_t lds = size_t(m.max_group) * nblk * 9u * 4u + size_t(m.iters) * rpi * m.max_group * 4u;
+    const size_t lds = (ActLds<Unit>::words(m.max_group * nunit) + size_t(m.iters) * rpi * m.max_group) * 4u;
     switch (lpr) {
         case 64: moe_matvec_kernel<Unit, MODE, 64><<<grid, 256, lds, s>>>(m); break;
         case 32: moe_matvec_kernel<Unit, MODE, 32><<<grid, 256, lds, s>>>(m); break;

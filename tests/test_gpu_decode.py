@@ -187,6 +187,13 @@ def test_expert_stages_against_fp64(moe, layer, orc, gpu_ctx, stream, gu_fmt, dn
     _within(gu.host(b_p, np.float32).reshape(N, d), parts, pm, "down parts")
 
 
+@pytest.mark.parametrize("gu_fmt,dn_fmt,d,I", [(1, 3, 4096, 256), (2, 1, 256, 4096)])
+def test_expert_stages_widest_and_narrowest_rows(moe, layer, orc, gpu_ctx, stream, gu_fmt, dn_fmt, d, I):
+    """The staged activation units at their most per workgroup (8 entries of 4096 values, 53 KB of
+    LDS) and at one unit per row."""
+    test_expert_stages_against_fp64(moe, layer, orc, gpu_ctx, stream, gu_fmt, dn_fmt, d, I)
+
+
 def test_null_expert_and_damaged_plan(moe, layer, orc, gpu_ctx, stream):
     print("case decode failure paths", flush=True)
     cfg = _small(layer, moe)

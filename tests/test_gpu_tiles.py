@@ -3,8 +3,9 @@
 Every group here is below 128 entries, so both expert stages run on the tile kernels; the
 shapes cover Q4_K, Q2_K and Q8_0 weights on both stages, reductions of one to five
 256-value slabs (activation slabs resident or streamed), one to eight column tiles per work
-item, a down reduction of 384 values, which ends with half a slab, and more gate/up items than workgroups (items run back to back), and few row tiles split over the workgroups. Each case checks every token of both stages and
-the layer against the CPU oracle with the benchmark configurations' bars (gate/up within
+item, a down reduction of 384 values, which ends with half a slab, more gate/up items than
+workgroups (items run back to back), and few row tiles split over the workgroups. Each case
+checks every token of both stages and the layer against the CPU oracle with the benchmark configurations' bars (gate/up within
 1 F16 ulp, down parts within 2e-5 + 2e-5 |x|, layer max-abs 2e-2 and rel-L2 5e-3), and the failure
 paths (a missing expert address zeroes that group's rows, leaves every other row as the clean
 run wrote it, and sets status bit 0; a broken
