@@ -12,6 +12,8 @@
 #include <stddef.h>
 #include <stdint.h>
 
+#include <type_traits>
+
 #include "sm_device.h"
 #include "sm_launch.h"
 #include "sm_topk.h"
@@ -621,8 +623,11 @@ __device__ __forceinline__ void gate_logit_block(const DenseDecode& m) {
 }
 
 // Workgroup bx of nb of one dense mat-vec (a launch of its own, or one part of a fused launch),
-// x_lds its dynamic LDS.
-template <int WT, bool GATE_UP, bool XF32, uint32_t LPR>
+// x_lds its dynamic LDS. NT: the activation rows (1, 2, 4 or 8: the power of two covering them;
+// a row past the last one repeats row 0 and is not stored), so that a chunk's rows are read from
+// LDS together: with a row count known only at run time each of them was a branch and a wait of
+// its own, 80 of them for a router row at T = 8.
+template <int WT, bool GATE_UP, bool XF32, uint32_t LPR, uint32_t NT>
 __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t bx, uint32_t nb, uint8_t* x_lds) {
     if (GATE_UP && m.gv != nullptr && bx == nb - 1u) {
         gate_logit_block<WT>(m);  // the job's last workgroup
@@ -663,11 +668,14 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
     const uint32_t row = matvec_rows_per_block(LPR) * bx + wave * RPW + lane / LPR;
     const bool row_ok = row < m.n_out;  // uniform within each LPR-lane segment
     const uint32_t wbytes = WT == kWF32 ? 4u : 2u;
-    float acc[NW][8];
+    float acc[NW][NT];
 #pragma unroll
     for (uint32_t w = 0; w < NW; ++w)
 #pragma unroll
-        for (uint32_t t = 0; t < 8u; ++t) acc[w][t] = 0.0f;
+        for (uint32_t t = 0; t < NT; ++t) acc[w][t] = 0.0f;
+    uint32_t xrow[NT];  // first value of each activation row
+#pragma unroll
+    for (uint32_t t = 0; t < NT; ++t) xrow[t] = t < m.rows ? t * m.k : 0u;
     const uint8_t* wr[2] = {m.w0 + uint64_t(row_ok ? row : 0u) * m.k * wbytes,
                             GATE_UP ? m.w1 + uint64_t(row_ok ? row : 0u) * m.k * wbytes : nullptr};
     // Chunks in flight per lane (at most): ten for the router's F32 rows, eight for F16/BF16
@@ -711,11 +719,10 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
                         }
                     }
 #pragma unroll
-                for (uint32_t t = 0; t < 8u; ++t) {
-                    if (t >= m.rows) break;
+                for (uint32_t t = 0; t < NT; ++t) {
                     float xv[VPC];
                     if (XF32) {
-                        const float* xp = reinterpret_cast<const float*>(x_lds) + t * m.k + VPC * c;
+                        const float* xp = reinterpret_cast<const float*>(x_lds) + xrow[t] + VPC * c;
                         const float4v a = *reinterpret_cast<const float4v*>(xp);
 #pragma unroll
                         for (uint32_t j = 0; j < 4u; ++j) xv[j] = a[j];
@@ -725,7 +732,7 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
                             for (uint32_t j = 0; j < 4u; ++j) xv[(4u + j) % VPC] = b[j];
                         }
                     } else {
-                        const uint8_t* xp = x_lds + (t * m.k + VPC * c) * 2u;
+                        const uint8_t* xp = x_lds + (xrow[t] + VPC * c) * 2u;
                         if (VPC == 8u) {
                             const u32x4 q = *reinterpret_cast<const u32x4*>(xp);
 #pragma unroll
@@ -752,34 +759,33 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
 #pragma unroll
     for (uint32_t w = 0; w < NW; ++w)
 #pragma unroll
-        for (uint32_t t = 0; t < 8u; ++t)
-            if (t < m.rows)
+        for (uint32_t t = 0; t < NT; ++t)
 #pragma unroll
-                for (uint32_t o = LPR / 2u; o > 0u; o >>= 1) acc[w][t] = acc[w][t] + __shfl_xor(acc[w][t], int(o));
+            for (uint32_t o = LPR / 2u; o > 0u; o >>= 1) acc[w][t] = acc[w][t] + __shfl_xor(acc[w][t], int(o));
     if (row_ok && lane % LPR == 0u) {
         const float b = (!GATE_UP && m.bias != nullptr) ? m.bias[row] : 0.0f;
 #pragma unroll
-        for (uint32_t t = 0; t < 8u; ++t)
+        for (uint32_t t = 0; t < NT; ++t)
             if (t < m.rows)
                 m.out[uint64_t(t) * m.n_out + row] = GATE_UP ? silu(acc[0][t]) * acc[NW - 1][t] : acc[0][t] + b;
     }
 }
 
-template <int WT, bool GATE_UP, bool XF32, uint32_t LPR>
+template <int WT, bool GATE_UP, bool XF32, uint32_t LPR, uint32_t NT>
 __global__ __launch_bounds__(256) void dense_decode_kernel(DenseDecode m) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t x_lds[];
-    dense_decode_body<WT, GATE_UP, XF32, LPR>(m, blockIdx.x, gridDim.x, x_lds);
+    dense_decode_body<WT, GATE_UP, XF32, LPR, NT>(m, blockIdx.x, gridDim.x, x_lds);
 }
 
 // The decode layer's router (F32 rows, with its snapshot copies) and its shared expert's gate/up
 // (F16/BF16 rows, with the gate logit) in one launch: both read only the layer's F16 input
 // rows, staged alike, and neither reads what the other writes. Workgroups [0, r_blocks) are the
 // router's, the rest the shared gate/up's.
-template <int WT, uint32_t LPR>
+template <int WT, uint32_t LPR, uint32_t NT>
 __global__ __launch_bounds__(256) void router_shared_decode_kernel(DenseDecode r, DenseDecode g, uint32_t r_blocks) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t x_lds[];
-    if (blockIdx.x < r_blocks) dense_decode_body<kWF32, false, false, LPR>(r, blockIdx.x, r_blocks, x_lds);
-    else dense_decode_body<WT, true, false, LPR>(g, blockIdx.x - r_blocks, gridDim.x - r_blocks, x_lds);
+    if (blockIdx.x < r_blocks) dense_decode_body<kWF32, false, false, LPR, NT>(r, blockIdx.x, r_blocks, x_lds);
+    else dense_decode_body<WT, true, false, LPR, NT>(g, blockIdx.x - r_blocks, gridDim.x - r_blocks, x_lds);
 }
 
 // A decode layer's front launch after the router: the plan (workgroup 0; with a.logits, the
@@ -787,7 +793,7 @@ __global__ __launch_bounds__(256) void router_shared_decode_kernel(DenseDecode r
 // rows (the next q_blocks workgroups, 256 values each) and the shared expert's down mat-vec
 // (the remaining workgroups, F32 hidden rows; WT < 0: none). None of the three reads what
 // another writes.
-template <int WT, uint32_t LPR>
+template <int WT, uint32_t LPR, uint32_t NT>
 __global__ __launch_bounds__(256) void decode_front_kernel(DecodePlanArgs a, const _Float16* x, uint8_t* y, uint32_t n,
                                                            uint32_t q_blocks, DenseDecode sd) {
     extern __shared__ __attribute__((aligned(1024))) uint8_t x_lds[];
@@ -818,7 +824,7 @@ __global__ __launch_bounds__(256) void decode_front_kernel(DecodePlanArgs a, con
     }
     if constexpr (WT >= 0) {
         const uint32_t first = 1u + q_blocks;
-        dense_decode_body<WT, false, true, LPR>(sd, blockIdx.x - first, gridDim.x - first, x_lds);
+        dense_decode_body<WT, false, true, LPR, NT>(sd, blockIdx.x - first, gridDim.x - first, x_lds);
     }
 }
 
@@ -828,6 +834,23 @@ __host__ __device__ constexpr uint32_t dense_lpr(uint32_t k, uint32_t vpc) {
     uint32_t lpr = 8;
     while (lpr < 64u && (k / vpc + lpr - 1u) / lpr > kPerLane) lpr <<= 1;
     return lpr;
+}
+
+// Calls f with the row count's NT and the LPR as constants.
+template <class F>
+hipError_t with_dense_shape(uint32_t rows, uint32_t lpr, F f) {
+    auto with_nt = [&](auto lpr_c) {
+        if (rows > 4u) return f(lpr_c, std::integral_constant<uint32_t, 8>());
+        if (rows > 2u) return f(lpr_c, std::integral_constant<uint32_t, 4>());
+        if (rows > 1u) return f(lpr_c, std::integral_constant<uint32_t, 2>());
+        return f(lpr_c, std::integral_constant<uint32_t, 1>());
+    };
+    switch (lpr) {
+        case 64: return with_nt(std::integral_constant<uint32_t, 64>());
+        case 32: return with_nt(std::integral_constant<uint32_t, 32>());
+        case 16: return with_nt(std::integral_constant<uint32_t, 16>());
+        default: return with_nt(std::integral_constant<uint32_t, 8>());
+    }
 }
 
 // Workgroups of one dense job: its row blocks, then the gate-logit workgroup (gate/up with a
@@ -858,12 +881,7 @@ hipError_t launch_dense_decode_t(const DenseDecode& m, hipStream_t s) {
         kern<<<grid, 256, lds, s>>>(mm);
         return hipGetLastError();
     };
-    switch (lpr) {
-        case 64: return go(dense_decode_kernel<WT, GATE_UP, XF32, 64>);
-        case 32: return go(dense_decode_kernel<WT, GATE_UP, XF32, 32>);
-        case 16: return go(dense_decode_kernel<WT, GATE_UP, XF32, 16>);
-        default: return go(dense_decode_kernel<WT, GATE_UP, XF32, 8>);
-    }
+    return with_dense_shape(m.rows, lpr, [&](auto l, auto nt) { return go(dense_decode_kernel<WT, GATE_UP, XF32, l.value, nt.value>); });
 }
 
 // ---- post ops ----------------------------------------------------------------------------
@@ -975,14 +993,9 @@ hipError_t launch_front_t(const DecodePlanArgs& a, const _Float16* x, uint8_t* y
         return hipGetLastError();
     };
     if constexpr (WT < 0) {
-        return go(decode_front_kernel<-1, 8>);
+        return go(decode_front_kernel<-1, 8, 1>);
     } else {
-        switch (lpr) {
-            case 64: return go(decode_front_kernel<WT, 64>);
-            case 32: return go(decode_front_kernel<WT, 32>);
-            case 16: return go(decode_front_kernel<WT, 16>);
-            default: return go(decode_front_kernel<WT, 8>);
-        }
+        return with_dense_shape(rows, lpr, [&](auto l, auto nt) { return go(decode_front_kernel<WT, l.value, nt.value>); });
     }
 }
 }  // namespace
@@ -1075,12 +1088,7 @@ hipError_t launch_router_shared_t(DenseDecode r, DenseDecode g, uint32_t lpr, hi
         kern<<<rb + gb, 256, lds, s>>>(r, g, rb);
         return hipGetLastError();
     };
-    switch (lpr) {
-        case 64: return go(router_shared_decode_kernel<WT, 64>);
-        case 32: return go(router_shared_decode_kernel<WT, 32>);
-        case 16: return go(router_shared_decode_kernel<WT, 16>);
-        default: return go(router_shared_decode_kernel<WT, 8>);
-    }
+    return with_dense_shape(r.rows, lpr, [&](auto l, auto nt) { return go(router_shared_decode_kernel<WT, l.value, nt.value>); });
 }
 }  // namespace
 
