@@ -163,9 +163,14 @@ static_assert(sizeof(DecodePlan) == 1620, "MoePlan layout");
 // first appearances; its slot is the group's start plus the number of earlier entries with
 // the same expert. The groups' starts are a prefix sum of their sizes in first-appearance
 // order. An id outside [0, E) sets status bit 1 and leaves an empty plan (n_groups = 0).
-// ids_lds (may be null): the route ids, already in LDS.
+// ids_lds (may be null): the route ids, already in LDS, in range and distinct within each token
+// (the top-k's own): each expert's tokens then make an 8-bit mask in LDS, which gives an entry's
+// rank and its group's size without a walk over the entries (two loops of up to 80 dependent
+// LDS reads each).
 __device__ __forceinline__ void moe_plan_body(const DecodePlanArgs& a, const int32_t* ids_lds = nullptr) {
     __shared__ int32_t e_s[128];
+    __shared__ uint32_t tok_s[512];   // ids_lds: tokens of each expert
+    __shared__ int32_t start_e[512];  // ids_lds: the expert's group start
     __shared__ uint32_t mask_s[2][2];
     __shared__ uint32_t size_w[2];
     __shared__ int32_t gstart_s[81], gidx_s[128];
@@ -178,20 +183,35 @@ __device__ __forceinline__ void moe_plan_body(const DecodePlanArgs& a, const int
         if (a.status != nullptr) *a.status = 0u;  // the stage's status word starts clear
     }
     const int32_t e = tid < n ? (ids_lds != nullptr ? ids_lds[tid] : a.ids[tid]) : -1;
-    if (tid < 128u) e_s[tid] = e;  // a 256-thread workgroup (the fused front launch) runs it too
-    __syncthreads();
-    if (tid < n && (e < 0 || uint32_t(e) >= a.n_experts)) atomicOr(&bad_s, 1u);
-    __syncthreads();
-    const bool bad = bad_s != 0u;
+    bool bad = false;
     uint32_t first = tid, rank = 0, size = 0;
-    if (tid < n) {
-        for (uint32_t j = 0; j < tid; ++j)
-            if (e_s[j] == e) {
-                if (first == tid) first = j;
-                ++rank;
-            }
-        if (first == tid)
-            for (uint32_t j = tid; j < n; ++j) size += e_s[j] == e ? 1u : 0u;
+    if (ids_lds != nullptr) {
+        for (uint32_t i = tid; i < 512u; i += blockDim.x) tok_s[i] = 0u;
+        __syncthreads();
+        const uint32_t tok = tid / a.top_k;
+        if (tid < n) atomicOr(&tok_s[e], 1u << tok);
+        __syncthreads();
+        if (tid < n) {
+            const uint32_t mask = tok_s[e];
+            rank = uint32_t(__builtin_popcount(mask & ((1u << tok) - 1u)));
+            size = uint32_t(__builtin_popcount(mask));
+            if (rank != 0u) first = ~0u;  // not the first; found by expert below
+        }
+    } else {
+        if (tid < 128u) e_s[tid] = e;  // a 256-thread workgroup (the fused front launch) runs it too
+        __syncthreads();
+        if (tid < n && (e < 0 || uint32_t(e) >= a.n_experts)) atomicOr(&bad_s, 1u);
+        __syncthreads();
+        bad = bad_s != 0u;
+        if (tid < n) {
+            for (uint32_t j = 0; j < tid; ++j)
+                if (e_s[j] == e) {
+                    if (first == tid) first = j;
+                    ++rank;
+                }
+            if (first == tid)
+                for (uint32_t j = tid; j < n; ++j) size += e_s[j] == e ? 1u : 0u;
+        }
     }
     const bool is_first = !bad && tid < n && first == tid;
     // Group index of a first appearance: first appearances before it (ballot prefix).
@@ -228,6 +248,7 @@ __device__ __forceinline__ void moe_plan_body(const DecodePlanArgs& a, const int
     if (is_first) {
         gidx_s[tid] = int32_t(gi);
         gstart_s[gi] = int32_t(start);
+        if (ids_lds != nullptr) start_e[e] = int32_t(start);
         const bool resident = a.resident == nullptr || a.resident[e] >= 0;
         P->grp_e[gi] = e;
         P->grp_start[gi] = int32_t(start);
@@ -244,7 +265,7 @@ __device__ __forceinline__ void moe_plan_body(const DecodePlanArgs& a, const int
         if (bad && a.status != nullptr) atomicOr(a.status, 2u);
     }
     if (!bad && tid < n) {
-        const uint32_t slot = uint32_t(gstart_s[gidx_s[first]]) + rank;
+        const uint32_t slot = uint32_t(ids_lds != nullptr ? start_e[e] : gstart_s[gidx_s[first]]) + rank;
         P->ent_dst[slot] = int32_t(tid);
         P->ent_tok[slot] = int32_t(tid / a.top_k);
         // Tiered mode: one use per entry (exact in F32 below 2^24).
@@ -802,15 +823,17 @@ __global__ __launch_bounds__(256) void decode_front_kernel(DecodePlanArgs a, con
             moe_plan_body(a);
             return;
         }
-        // The route first: up to 4 tokens one per wave, up to 8 two per wave (slots for E <= 512).
+        // The route first, tokens w and w + 4 on wave w (slots for E <= 512).
         __shared__ int32_t ids_s[80];
+        __shared__ uint2 cand[4][kTopkCand];
         const uint32_t wave = threadIdx.x >> 6;
-        if (a.rows <= 4u)
-            topk_token<8, true>(a.logits, a.route_ids, a.route_weights, a.rows, a.n_experts, a.top_k, 0, nullptr, wave,
-                                ids_s);
-        else
-            topk_token<16, false>(a.logits, a.route_ids, a.route_weights, a.rows, a.n_experts, a.top_k, 0, nullptr,
-                                  threadIdx.x >> 5, ids_s);
+        float v[8], v4[8];
+        topk_load(a.logits, a.rows, a.n_experts, wave, v);
+        if (NT > 4u) topk_load(a.logits, a.rows, a.n_experts, wave + 4u, v4);
+        topk_token(v, a.route_ids, a.route_weights, a.rows, a.n_experts, a.top_k, 0, nullptr, wave, cand[wave], ids_s);
+        if (NT > 4u)
+            topk_token(v4, a.route_ids, a.route_weights, a.rows, a.n_experts, a.top_k, 0, nullptr, wave + 4u, cand[wave],
+                       ids_s);
         __syncthreads();
         moe_plan_body(a, ids_s);
         return;
@@ -993,7 +1016,7 @@ hipError_t launch_front_t(const DecodePlanArgs& a, const _Float16* x, uint8_t* y
         return hipGetLastError();
     };
     if constexpr (WT < 0) {
-        return go(decode_front_kernel<-1, 8, 1>);
+        return rows > 4u ? go(decode_front_kernel<-1, 8, 8>) : go(decode_front_kernel<-1, 8, 1>);
     } else {
         return with_dense_shape(rows, lpr, [&](auto l, auto nt) { return go(decode_front_kernel<WT, l.value, nt.value>); });
     }

@@ -7,7 +7,6 @@
 namespace sm {
 namespace {
 
-constexpr uint32_t kTopkWaveRows = 1024;  // top-k: one token per wave up to this many tokens
 
 // ---------------------------------------------------------------------------------------
 // Router GEMM: logits[t,e] = sum_k x[t,k] * W[e,k], F16 activations, F32 weights.
@@ -218,14 +217,17 @@ __global__ __launch_bounds__(kRouterThreads) void router_gemm_kernel(const _Floa
     }
 }
 
-template <int NV, bool WAVE>
+template <int NV>
 __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict__ logits,
                                                          int32_t* __restrict__ ids,
                                                          float* __restrict__ weights,
                                                          uint32_t rows, uint32_t E, uint32_t K,
                                                          int divide, uint32_t* __restrict__ hist) {
-    const uint32_t t = WAVE ? blockIdx.x * 4u + (threadIdx.x >> 6) : blockIdx.x * 8u + (threadIdx.x >> 5);
-    topk_token<NV, WAVE>(logits, ids, weights, rows, E, K, divide, hist, t, nullptr);
+    __shared__ uint2 cand[4][kTopkCand];
+    const uint32_t wave = threadIdx.x >> 6, t = blockIdx.x * 4u + wave;
+    float v[NV];
+    topk_load(logits, rows, E, t, v);
+    topk_token(v, ids, weights, rows, E, K, divide, hist, t, cand[wave], nullptr);
 }
 
 // ---------------------------------------------------------------------------------------
@@ -727,22 +729,11 @@ hipError_t launch_router_gemm(const _Float16* x, const float* w, const float* bi
 hipError_t launch_route_topk(const float* logits, int32_t* ids, float* weights, uint32_t rows,
                              uint32_t E, uint32_t K, int divide, hipStream_t s, uint32_t* hist) {
     if (E == 0u || E > 512u || K == 0u || K > 32u || K > E) return hipErrorInvalidValue;
-    // Up to 1024 tokens (one wave per SIMD at most) a token takes a whole wave; more tokens
-    // share waves two by two.
-    if (rows <= kTopkWaveRows) {
-        const uint32_t blocks = (rows + 3u) / 4u, nv = (E + 63u) / 64u;
-        if (nv <= 1) route_topk_kernel<1, true><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-        else if (nv <= 2) route_topk_kernel<2, true><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-        else if (nv <= 4) route_topk_kernel<4, true><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-        else route_topk_kernel<8, true><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-    } else {
-        const uint32_t blocks = (rows + 7u) / 8u, nv = (E + 31u) / 32u;
-        if (nv <= 1) route_topk_kernel<1, false><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-        else if (nv <= 2) route_topk_kernel<2, false><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-        else if (nv <= 4) route_topk_kernel<4, false><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-        else if (nv <= 8) route_topk_kernel<8, false><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-        else route_topk_kernel<16, false><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-    }
+    const uint32_t blocks = (rows + 3u) / 4u, nv = (E + 63u) / 64u;
+    if (nv <= 1) route_topk_kernel<1><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
+    else if (nv <= 2) route_topk_kernel<2><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
+    else if (nv <= 4) route_topk_kernel<4><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
+    else route_topk_kernel<8><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
     return hipGetLastError();
 }
 
