@@ -661,6 +661,7 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
         const uint32_t w = (bx - m.row_blocks) * 256u + threadIdx.x;
         if (w < m.snap_words) m.snap_dst[w] = m.snap_src[w];
         else if (w - m.snap_words < m.snap_words2) m.snap_dst2[w - m.snap_words] = m.snap_src2[w - m.snap_words];
+        report_read(m.snap_done != nullptr ? m.snap_done + (bx - m.row_blocks) : nullptr, m.snap_value);
         return;
     }
     constexpr uint32_t RPW = 64u / LPR;
@@ -948,9 +949,10 @@ __global__ __launch_bounds__(256) void combine_decode_kernel(const float* parts,
 // Copies a validated address table (pinned host ring slot) into its device snapshot and clears
 // the stage's status word (a standalone expert stage, whose plan came from elsewhere).
 __global__ __launch_bounds__(256) void snapshot_copy_kernel(const uint64_t* src, uint64_t* dst, uint32_t words,
-                                                            uint32_t* status) {
+                                                            uint32_t* status, uint32_t* done, uint32_t done_value) {
     for (uint32_t w = threadIdx.x; w < words; w += 256u) dst[w] = src[w];
     if (threadIdx.x == 0 && status != nullptr) *status = 0u;
+    report_read(done, done_value);
 }
 
 template <class Unit, int MODE>
@@ -1045,8 +1047,9 @@ hipError_t launch_swiglu_q8_1(const float* gate, const float* up, float* hidden,
     return hipGetLastError();
 }
 
-hipError_t launch_snapshot_copy(const uint64_t* src, uint64_t* dst, uint32_t words, uint32_t* status, hipStream_t s) {
-    snapshot_copy_kernel<<<1, 256, 0, s>>>(src, dst, words, status);
+hipError_t launch_snapshot_copy(const uint64_t* src, uint64_t* dst, uint32_t words, uint32_t* status, uint32_t* done,
+                                uint32_t done_value, hipStream_t s) {
+    snapshot_copy_kernel<<<1, 256, 0, s>>>(src, dst, words, status, done, done_value);
     return hipGetLastError();
 }
 
@@ -1087,6 +1090,8 @@ DenseDecode router_job(const _Float16* x, const float* w, const float* bias, flo
     m.snap_src2 = snap.src2;
     m.snap_dst2 = snap.dst2;
     m.snap_words2 = snap.words2;
+    m.snap_done = snap.done;
+    m.snap_value = snap.done_value;
     m.w0 = reinterpret_cast<const uint8_t*>(w);
     m.x = x;
     m.bias = bias;

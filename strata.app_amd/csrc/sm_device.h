@@ -94,6 +94,15 @@ __device__ __forceinline__ uint32_t weight_fault(const uint8_t* w0, const uint8_
     return ((a | b) & 1u) ? 4u : 0u;
 }
 
+// Called by a whole workgroup once each of its threads has issued the stores of what it read from
+// a pinned host slot (a store is issued after its data has arrived): tells the host, through one
+// pinned word (may be null), that the slot may be written again.
+__device__ __forceinline__ void report_read(uint32_t* done, uint32_t value) {
+    __syncthreads();
+    if (done != nullptr && threadIdx.x == 0)
+        __hip_atomic_store(done, value, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_SYSTEM);
+}
+
 // Byte j (0..3) of a dword as an exact float (selected as v_cvt_f32_ubyte{j}).
 __device__ __forceinline__ float ubyte(uint32_t w, int j) { return float((w >> (8 * j)) & 0xffu); }
 

@@ -104,6 +104,8 @@ struct PlanCheck {
     uint32_t n_counters;
     uint32_t keep_status;       // non-zero: the status words are not cleared first (they
                                 // accumulate over the chunks of one prompt)
+    uint32_t* done;             // pinned host word (may be null) that gets done_value once the
+    uint32_t done_value;        // snapshot sources have been read
 };
 hipError_t launch_plan_validate(const PlanCheck& c, hipStream_t s);
 // The gather of a full layer with both expert stages' checks in the same launch: one extra
@@ -199,8 +201,10 @@ hipError_t launch_decode_plan(const DecodePlanArgs& a, hipStream_t s);
 // hidden = silu(gate) * up (F32, rows x n, n a multiple of 32) and its Q8_1 blocks y, one launch.
 hipError_t launch_swiglu_q8_1(const float* gate, const float* up, float* hidden, uint8_t* y, uint32_t n, uint32_t rows,
                               hipStream_t s);
-// A standalone expert stage's snapshot copy (src may be null: nothing copied); clears *status.
-hipError_t launch_snapshot_copy(const uint64_t* src, uint64_t* dst, uint32_t words, uint32_t* status, hipStream_t s);
+// A standalone expert stage's snapshot copy (src may be null: nothing copied); clears *status and
+// reports in *done (pinned host memory, may be null) once src has been read.
+hipError_t launch_snapshot_copy(const uint64_t* src, uint64_t* dst, uint32_t words, uint32_t* status, uint32_t* done,
+                                uint32_t done_value, hipStream_t s);
 // Q8_1 blocks (36 B: half d, half sum, int8 q[32]) of rows x n values (F16 or F32 input).
 hipError_t launch_quantize_q8_1(const void* x, bool f32_input, uint8_t* y, uint32_t n, uint32_t rows, hipStream_t s);
 // Grouped mat-vec of one stage over a MoePlan. gate/up: act = Q8_1 [rows][k/32] by token,
@@ -240,6 +244,8 @@ struct DenseDecode {
     const uint64_t* snap_src2;
     uint64_t* snap_dst2;
     uint32_t snap_words2;
+    uint32_t* snap_done;  // one pinned host word per copying workgroup (may be null) that gets
+    uint32_t snap_value;  // snap_value once the workgroup has read its share
     uint32_t row_blocks;  // set by the launcher
 };
 struct SnapshotCopy {
@@ -249,7 +255,11 @@ struct SnapshotCopy {
     const uint64_t* src2;
     uint64_t* dst2;
     uint32_t words2;
+    uint32_t* done;
+    uint32_t done_value;
 };
+// Workgroups that copy the tables of `c` in the decode router's launch (256 words each).
+inline uint32_t snapshot_copy_blocks(const SnapshotCopy& c) { return (c.words + c.words2 + 255u) / 256u; }
 hipError_t launch_dense_decode(Fmt fmt, bool gate_up, const DenseDecode& m, hipStream_t s);
 // The router of a decode layer (T <= 8 rows): logits[t][e] = x_t . W_e + bias[e] with F32
 // weights [E][d] and F32 accumulation (d a multiple of 64).

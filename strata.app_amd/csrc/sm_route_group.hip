@@ -512,7 +512,7 @@ __device__ __forceinline__ void check_plan(const PlanCheck& c, bool reset_status
                        p->grp_start[ng] == int32_t(N))
                           ? 1u : 0u;
     }
-    __syncthreads();
+    report_read(c.done, c.done_value);  // (its barrier also shows s_header_ok)
     if (!s_header_ok) {
         if (tid == 0) fail();
         return;

@@ -61,3 +61,36 @@ def test_two_streams_alternating_commits(moe, layer, gpu_ctx):
             assert dec[i].read_status() == 0
             assert np.array_equal(_out(pre[i]).view(np.uint32), want_pre[i].view(np.uint32)), (rnd, "prefill", i)
             assert np.array_equal(_out(dec[i]).view(np.uint32), want_dec[i].view(np.uint32)), (rnd, "decode", i)
+
+
+def test_ring_reuse_through_stage_entry_points(moe, layer, gpu_ctx, stream):
+    """The standalone stages report their slots from other kernels than the layers do: 80 commits
+    each of two workspaces' gate/up and routed-FFN stages, alternately, one slot per stage, so
+    every slot is handed out again several times."""
+    import torch
+    print("case ring reuse through standalone stages", flush=True)
+    pre = [layer.LayerWorkspace(gpu_ctx, c, layer.make_inputs(c)) for c in (_prefill(layer, moe, 0xC0C1A),
+                                                                            _prefill(layer, moe, 0xC0C1B))]
+    dec = [layer.DecodeWorkspace(gpu_ctx, c, layer.make_inputs(c)) for c in (_decode(layer, moe, 0xC0C1C),
+                                                                            _decode(layer, moe, 0xC0C1D))]
+    for p, d in zip(pre, dec):
+        p.run_layer(stream)
+        d.run(stream)
+    torch.cuda.synchronize()
+    outs = [b for p, d in zip(pre, dec) for b in (p.hidden, d.gate, d.parts)]
+    want = [gu.host(b, np.uint32).copy() for b in outs]
+    for b in outs:
+        b.tensor.fill_(7)
+    keep = []
+    for _ in range(80):
+        for p, d in zip(pre, dec):
+            keep = [p.gate_up_buffers(), d.routed_buffers()]
+            seg = gpu_ctx.segment()
+            ok, err = seg.encode_prefill_moe_gu(p.shape, p.cfg.gate_up_fmt, keep[0])
+            assert ok, err
+            ok, err = seg.encode_moe_routed_ffn(d.shape, d.cfg.gate_up_fmt, d.cfg.down_fmt, keep[1])
+            assert ok, err
+            seg.commit(stream)
+    torch.cuda.synchronize()
+    for b, w in zip(outs, want):
+        assert np.array_equal(gu.host(b, np.uint32), w)
