@@ -241,6 +241,8 @@ __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict
 //   scatter one 256-entry tile per workgroup: hist row += first slot (the reference's
 //           "cursor at tile start"); stable in-tile rank from per-wave ballot matching of
 //           the 9-bit ids plus the counts of earlier waves; src[slot] = i/k, dst[slot] = i
+// Up to 80 tiles one workgroup does the scan and the plan and leaves the final cursors
+// (group_plan_kernel); the gather then does the scatter's part.
 // ---------------------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void group_count_kernel(const int32_t* __restrict__ ids, uint32_t N,
                                                           uint32_t E, uint32_t* __restrict__ hist,
@@ -426,6 +428,138 @@ __global__ __launch_bounds__(kScanThreads) void group_scan_plan_kernel(uint32_t*
     }
 }
 
+// The column scan and the plan of up to 2 HELD histogram tiles in one workgroup: thread (half, e)
+// loads its half of column e whole and keeps it, so the counts are one round trip, no other
+// workgroup has to be waited for (the arrival of the kernel above is an agent-scope
+// acquire-release, which writes the XCD's L2 back), and the first slots are known before the
+// columns are written: hist rows get their final cursors here, and the gather, which recomputes
+// every entry's slot from them anyway, writes src and dst (its SCATTER form) instead of a
+// scatter launch. One scan carries count and group index, another tiles and misses.
+// The grouping's launches (events) at 1, 4, 21 and 80 tiles: 11.9 -> 6.0, 13.2 -> 6.0, 13.1 -> 8.9
+// and 14.2 -> 9.6 us, the gather unchanged within 0.4 us. 80 tiles is what a thread's registers
+// hold (40 counts each); longer columns are scanned by E / 32 workgroups.
+template <uint32_t HELD>
+__global__ __launch_bounds__(kScanThreads) void group_plan_kernel(uint32_t* __restrict__ hist, uint32_t E, uint32_t N,
+                                                                  uint32_t n_tiles, Plan* __restrict__ plan,
+                                                                  uint32_t* __restrict__ tiles, GroupPrep prep,
+                                                                  const int32_t* __restrict__ resident) {
+    __shared__ uint32_t s_part[512], s_lo[8], s_hi[8];
+    __shared__ uint32_t s_firstslot[512];              // by expert
+    __shared__ uint32_t s_ge[512], s_tstart[513], s_first[513];  // by group: expert | missing << 16, first tile, first slot
+    const uint32_t tid = threadIdx.x, lane = tid & 63u, e = tid & 511u, half = tid >> 9;
+    const uint32_t per = (n_tiles + 1u) >> 1, t_begin = half * per;
+    const uint32_t t_end = t_begin + per < n_tiles ? t_begin + per : n_tiles;
+    const bool col = e < E;
+    uint32_t hv[HELD];
+#pragma unroll
+    for (uint32_t j = 0; j < HELD; ++j) {  // clamped into the column, so no branch sits between the loads
+        const uint32_t t = t_begin + j < t_end ? t_begin + j : 0u;
+        hv[j] = hist[uint64_t(t) * E + (col ? e : 0u)];
+    }
+    const bool res = resident == nullptr || !col || resident[e] >= 0;
+    if (tid == 0) {
+        if (prep.status != nullptr) *prep.status = 0u;
+        if (prep.status2 != nullptr) *prep.status2 = 0u;
+    }
+    for (uint32_t i = tid; i < prep.clear_words; i += kScanThreads) prep.clear[i] = 0u;
+    uint32_t local = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < HELD; ++j) {
+        hv[j] = col && t_begin + j < t_end ? hv[j] : 0u;
+        local += hv[j];
+    }
+    if (half == 1u) s_part[e] = local;
+    __syncthreads();
+    const uint32_t count = local + (half == 0u ? s_part[e] : 0u);  // half 0: the column's total
+    if (half == 0u) s_part[e] = local;  // (read above by this thread alone) half 1's tiles follow these
+    // Packed inclusive scans over the experts (half 0's eight waves): count (at most
+    // 2 HELD * 256 < 2^16) | groups, and tiles | misses.
+    const uint32_t nt_e = (count + kExpertTile - 1u) / kExpertTile;
+    const uint32_t own_lo = half == 0u ? count | (count != 0u ? 1u << 16 : 0u) : 0u;
+    const uint32_t own_hi = half == 0u ? nt_e | (count != 0u && !res ? 1u << 16 : 0u) : 0u;
+    uint32_t lo = own_lo, hi = own_hi;
+    if (half == 0u) {
+#pragma unroll
+        for (uint32_t off = 1; off < 64u; off <<= 1) {
+            const uint32_t a = __shfl_up(lo, off), b = __shfl_up(hi, off);
+            if (lane >= off) {
+                lo += a;
+                hi += b;
+            }
+        }
+        if (lane == 63u) {
+            s_lo[tid >> 6] = lo;
+            s_hi[tid >> 6] = hi;
+        }
+    }
+    __syncthreads();
+    uint32_t all_lo = 0, all_hi = 0, before_lo = 0, before_hi = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < 8u; ++w) {
+        if (w < (tid >> 6)) {
+            before_lo += s_lo[w];
+            before_hi += s_hi[w];
+        }
+        all_lo += s_lo[w];
+        all_hi += s_hi[w];
+    }
+    const uint32_t total_count = all_lo & 0xffffu, total_groups = all_lo >> 16;
+    const uint32_t total_tiles = all_hi & 0xffffu, total_miss = all_hi >> 16;
+    if (half == 0u) {
+        const uint32_t ex_lo = before_lo + lo - own_lo, ex_hi = before_hi + hi - own_hi;  // exclusive
+        const uint32_t first = ex_lo & 0xffffu, grp = ex_lo >> 16;
+        s_firstslot[e] = first;
+        if (col) hist[uint64_t(n_tiles) * E + e] = first;
+        if (count != 0u) {
+            s_ge[grp] = e | (res ? 0u : 1u << 16);
+            s_tstart[grp] = ex_hi & 0xffffu;
+            s_first[grp] = first;
+        }
+    }
+    __syncthreads();
+    // The columns' final cursors: first slot + entries of the tiles before.
+    if (col) {
+        uint32_t run = s_firstslot[e] + (half == 1u ? s_part[e] : 0u);
+#pragma unroll
+        for (uint32_t j = 0; j < HELD; ++j)
+            if (t_begin + j < t_end) {
+                hist[uint64_t(t_begin + j) * E + e] = run;
+                run += hv[j];
+            }
+    }
+    // The whole 6400-byte slot, each word once (unused group slots -1 / 0, tail zero).
+    uint32_t* words = reinterpret_cast<uint32_t*>(plan);
+    for (uint32_t i = tid; i < kPlanSlotBytes / 4; i += kScanThreads) {
+        uint32_t val = 0;
+        if (i < 8u) {
+            val = i == 0u ? total_groups : i == 1u ? N : i == 2u ? total_miss : i == 3u ? (total_miss == 0u ? 1u : 0u)
+                : i == 4u ? total_tiles : i == 5u ? N - total_count : 0u;
+        } else if (i < 8u + 512u) {
+            val = i - 8u < total_groups ? s_ge[i - 8u] & 0xffffu : 0xffffffffu;
+        } else if (i < 8u + 1024u) {
+            val = i - 520u < total_groups ? 1u - (s_ge[i - 520u] >> 16) : 0xffffffffu;
+        } else if (i < 8u + 1024u + 513u) {
+            const uint32_t g = i - 1032u;
+            val = g < total_groups ? s_first[g] : g == total_groups ? total_count : 0u;
+        }
+        words[i] = val;
+    }
+    // Every group has at least one tile, so the groups' first tiles ascend strictly.
+    for (uint32_t i = tid; i < total_tiles; i += kScanThreads) {
+        uint32_t lo_g = 0, hi_g = total_groups;
+        while (hi_g - lo_g > 1u) {
+            const uint32_t mid = (lo_g + hi_g) >> 1;
+            if (s_tstart[mid] <= i) lo_g = mid;
+            else hi_g = mid;
+        }
+        tiles[2 * i] = lo_g;
+        tiles[2 * i + 1] = s_first[lo_g] + kExpertTile * (i - s_tstart[lo_g]);
+    }
+}
+constexpr uint32_t kPlanHeld = 8, kPlanHeldMax = 40;
+// Whether the grouping of n_tiles histogram tiles runs in one workgroup.
+constexpr bool grouping_in_one(uint32_t n_tiles) { return n_tiles <= 2u * kPlanHeldMax; }
+
 __global__ __launch_bounds__(256) void group_scatter_kernel(const int32_t* __restrict__ ids, uint32_t N,
                                                             uint32_t K, uint32_t E, uint32_t n_tiles,
                                                             uint32_t* __restrict__ hist,
@@ -579,14 +713,18 @@ __global__ __launch_bounds__(512) void plan_validate_kernel(PlanCheck c) {
 // workgroup (tile, part) also marks its share of the tile's entries of `dst` in the bitset,
 // which is the reference's destination check (prefill_moe_down_dispatch.mm:470-520) spread
 // over the gather: an entry outside [0, N) or one already marked sets bit 1 of the down status.
+// SCATTER (the grouping ran in one workgroup, no scatter launch): the workgroups of part 0 also
+// write src and dst, and where the checked destinations are that dst, a workgroup marks its
+// share of the tile's slots instead (the slots are a permutation exactly if dst is).
 constexpr uint32_t kGatherPart = 16, kGatherBatch = 2;
-template <bool CHECK>
+template <bool CHECK, bool SCATTER>
 __global__ __launch_bounds__(256) void gather_kernel(const u32x4* __restrict__ x, uint32_t vpr,
                                                      const int32_t* __restrict__ ids,
                                                      const uint32_t* __restrict__ hist, uint32_t K, uint32_t E,
                                                      uint32_t parts, const Plan* __restrict__ plan, uint32_t N,
-                                                     u32x4* __restrict__ xs, PlanCheck c,
-                                                     const int32_t* __restrict__ dst, uint32_t* __restrict__ bits) {
+                                                     u32x4* __restrict__ xs, PlanCheck c, const int32_t* check_dst,
+                                                     uint32_t* __restrict__ bits, int32_t* __restrict__ src,
+                                                     int32_t* dst) {
     __shared__ uint32_t wcnt[4][512];
     __shared__ uint32_t s_base[512];
     __shared__ uint32_t s_slot[kCountTile];
@@ -618,19 +756,21 @@ __global__ __launch_bounds__(256) void gather_kernel(const u32x4* __restrict__ x
     const uint64_t entry = uint64_t(i0) + tid;
     const int32_t id = entry < N ? ids[entry] : -1;  // issued before the plan reads
     for (uint32_t e = tid; e < E; e += 256u) s_base[e] = hist[uint64_t(tile) * E + e];
+    const uint32_t ng = plan->n_groups, p_entries = plan->n_entries, p_bad = plan->bad;
     // CHECK: this workgroup's share of the tile's destinations, loaded with the other first
     // loads and marked after the copies (a returning atomic would hold the copies behind its
     // round trip).
+    const uint32_t per = (kCountTile + parts - 1u) / parts;
+    const bool by_slot = SCATTER && check_dst == dst;
     bool marks = false;
     uint32_t dv = 0;
-    if constexpr (CHECK) {
-        const uint32_t per = (kCountTile + parts - 1u) / parts;
+    if (CHECK && !by_slot) {
         const uint32_t i = i0 + part * per + tid;
         marks = tid < per && i < i1;
-        if (marks) dv = uint32_t(dst[i]);
+        if (marks) dv = uint32_t(check_dst[i]);
     }
     auto mark = [&]() {
-        if (!marks) return;
+        if (!CHECK || !marks) return;
         if (dv >= N) {
             atomicOr(c.status2, 2u);
         } else {
@@ -639,17 +779,7 @@ __global__ __launch_bounds__(256) void gather_kernel(const u32x4* __restrict__ x
         }
     };
     for (uint32_t k = tid; k < 4u * 512u; k += 256u) (&wcnt[0][0])[k] = 0u;
-    const uint32_t ng = plan->n_groups;
-    if (ng > 512u || plan->n_entries != N || plan->bad > plan->n_entries) {
-        mark();
-        return;
-    }
-    const int32_t sorted_signed = plan->grp_start[ng];
-    if (sorted_signed < 0 || uint32_t(sorted_signed) != N - plan->bad) {
-        mark();
-        return;
-    }
-    // The entry's slot, as group_scatter_kernel computed it.
+    // The entry's slot, as group_scatter_kernel computes it.
     const bool valid = id >= 0 && uint32_t(id) < E;
     const uint32_t key = valid ? uint32_t(id) : 1023u;
     uint64_t match = ~0ull;
@@ -661,6 +791,8 @@ __global__ __launch_bounds__(256) void gather_kernel(const u32x4* __restrict__ x
     }
     const uint32_t rank = __popcll(match & ((1ull << lane) - 1ull));
     const uint64_t gt = lane == 63u ? 0ull : (~0ull << (lane + 1u));
+    // The plan header's second look-up travels while the slots are computed.
+    const int32_t sorted_signed = plan->grp_start[ng <= 512u ? ng : 0u];
     __syncthreads();
     if (valid && (match & gt) == 0ull) wcnt[wave][id] = rank + 1u;
     __syncthreads();
@@ -668,9 +800,24 @@ __global__ __launch_bounds__(256) void gather_kernel(const u32x4* __restrict__ x
     if (valid) {
         slot = s_base[id] + rank;
         for (uint32_t w = 0; w < wave; ++w) slot += wcnt[w][id];
-        if (slot >= uint32_t(sorted_signed)) slot = ~0u;  // only behind an inconsistent histogram
+        if (slot >= N) slot = ~0u;  // only behind an inconsistent histogram
     }
-    s_slot[tid] = slot;
+    if (SCATTER) {
+        if (part == 0u && slot != ~0u) {
+            src[slot] = int32_t(entry / K);
+            dst[slot] = int32_t(entry);
+        }
+        if (CHECK && by_slot) {
+            marks = entry < N && tid / per == part;
+            dv = slot;
+        }
+    }
+    if (ng > 512u || p_entries != N || p_bad > p_entries || sorted_signed < 0 ||
+        uint32_t(sorted_signed) != N - p_bad) {  // uniform
+        mark();
+        return;
+    }
+    s_slot[tid] = slot < uint32_t(sorted_signed) ? slot : ~0u;
     __syncthreads();
     for (uint32_t tb = t0;; tb += kGatherBatch * rpar) {
         if (tb != t0) load_batch(tb);
@@ -745,32 +892,44 @@ hipError_t launch_grouping(const int32_t* ids, uint32_t rows, uint32_t K, uint32
     const uint32_t n_tiles = (N + kCountTile - 1) / kCountTile;
     uint32_t* arrive = reinterpret_cast<uint32_t*>(reinterpret_cast<uint8_t*>(plan) + kArriveBytes);
     if (!counted) group_count_kernel<<<n_tiles, 256, 0, s>>>(ids, N, E, hist, arrive);
-    group_scan_plan_kernel<<<(E + 31) / 32, kScanThreads, 0, s>>>(hist, E, N, n_tiles, plan, tiles, arrive,
-                                                                  prep != nullptr ? *prep : GroupPrep{}, resident);
+    const GroupPrep p = prep != nullptr ? *prep : GroupPrep{};
+    if (grouping_in_one(n_tiles)) {  // the gather writes src and dst
+        if (n_tiles <= 2u * kPlanHeld)
+            group_plan_kernel<kPlanHeld><<<1, kScanThreads, 0, s>>>(hist, E, N, n_tiles, plan, tiles, p, resident);
+        else
+            group_plan_kernel<kPlanHeldMax><<<1, kScanThreads, 0, s>>>(hist, E, N, n_tiles, plan, tiles, p, resident);
+        return hipGetLastError();
+    }
+    group_scan_plan_kernel<<<(E + 31) / 32, kScanThreads, 0, s>>>(hist, E, N, n_tiles, plan, tiles, arrive, p, resident);
     group_scatter_kernel<<<n_tiles, 256, 0, s>>>(ids, N, K, E, n_tiles, hist, src, dst);
     return hipGetLastError();
 }
 
 hipError_t launch_gather(const _Float16* x, uint32_t d, const int32_t* ids, const uint32_t* hist, uint32_t K,
-                         uint32_t E, const Plan* plan, uint32_t N, _Float16* xs, hipStream_t s) {
+                         uint32_t E, const Plan* plan, uint32_t N, _Float16* xs, int32_t* src, int32_t* dst,
+                         hipStream_t s) {
     const uint32_t vpr = d / 8, parts = vpr / kGatherPart;  // d % 256 == 0
-    const uint32_t blocks = parts * ((N + kCountTile - 1) / kCountTile);  // (tile, part) pairs
-    gather_kernel<false><<<blocks, 256, 0, s>>>(reinterpret_cast<const u32x4*>(x), vpr, ids, hist, K, E, parts,
-                                                plan, N, reinterpret_cast<u32x4*>(xs), PlanCheck{}, nullptr, nullptr);
-    return hipGetLastError();
+    const uint32_t n_tiles = (N + kCountTile - 1) / kCountTile;
+    auto go = [&](auto kern) {
+        kern<<<parts * n_tiles, 256, 0, s>>>(reinterpret_cast<const u32x4*>(x), vpr, ids, hist, K, E, parts, plan, N,
+                                             reinterpret_cast<u32x4*>(xs), PlanCheck{}, nullptr, nullptr, src, dst);
+        return hipGetLastError();
+    };
+    return grouping_in_one(n_tiles) ? go(gather_kernel<false, true>) : go(gather_kernel<false, false>);
 }
-
 hipError_t launch_gather_checked(const _Float16* x, uint32_t d, const int32_t* ids, const uint32_t* hist, uint32_t K,
-                                 uint32_t E, const Plan* plan, uint32_t N, _Float16* xs, const PlanCheck& c,
-                                 const int32_t* dst, uint32_t* bits, hipStream_t s) {
+                                 uint32_t E, const Plan* plan, uint32_t N, _Float16* xs, int32_t* src, int32_t* dst,
+                                 const PlanCheck& c, const int32_t* check_dst, uint32_t* bits, hipStream_t s) {
     if (c.snap_words > 1536u || c.snap_words2 > 1536u || c.status2 == nullptr) return hipErrorInvalidValue;
     const uint32_t vpr = d / 8, parts = vpr / kGatherPart;
-    const uint32_t blocks = 1u + parts * ((N + kCountTile - 1) / kCountTile);  // check + copy workgroups
-    gather_kernel<true><<<blocks, 256, 0, s>>>(reinterpret_cast<const u32x4*>(x), vpr, ids, hist, K, E, parts, plan,
-                                               N, reinterpret_cast<u32x4*>(xs), c, dst, bits);
-    return hipGetLastError();
+    const uint32_t n_tiles = (N + kCountTile - 1) / kCountTile;
+    auto go = [&](auto kern) {  // check + copy workgroups
+        kern<<<1u + parts * n_tiles, 256, 0, s>>>(reinterpret_cast<const u32x4*>(x), vpr, ids, hist, K, E, parts, plan,
+                                                  N, reinterpret_cast<u32x4*>(xs), c, check_dst, bits, src, dst);
+        return hipGetLastError();
+    };
+    return grouping_in_one(n_tiles) ? go(gather_kernel<true, true>) : go(gather_kernel<true, false>);
 }
-
 hipError_t launch_plan_validate(const PlanCheck& c, hipStream_t s) {
     if (c.snap_words > 1536u || c.snap_words2 > 1536u) return hipErrorInvalidValue;  // E <= 512
     const uint32_t blocks = 1u + c.clear_words / (512u * 16u);

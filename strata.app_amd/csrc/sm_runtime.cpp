@@ -374,7 +374,8 @@ void encode_grouping_launch(sm_segment* seg, const sm_moe_shape& s, const GroupR
                                      reinterpret_cast<const int32_t*>(r.ids),
                                      reinterpret_cast<const uint32_t*>(r.hist), K, E,
                                      reinterpret_cast<const sm::Plan*>(r.plan), rows * K,
-                                     reinterpret_cast<_Float16*>(r.gathered), st);
+                                     reinterpret_cast<_Float16*>(r.gathered), reinterpret_cast<int32_t*>(r.src),
+                                     reinterpret_cast<int32_t*>(r.dst), st);
         });
         return;
     }
@@ -384,7 +385,8 @@ void encode_grouping_launch(sm_segment* seg, const sm_moe_shape& s, const GroupR
                                          reinterpret_cast<const int32_t*>(r.ids),
                                          reinterpret_cast<const uint32_t*>(r.hist), K, E,
                                          reinterpret_cast<const sm::Plan*>(r.plan), rows * K,
-                                         reinterpret_cast<_Float16*>(r.gathered), l.check, l.dst, l.bits, st);
+                                         reinterpret_cast<_Float16*>(r.gathered), reinterpret_cast<int32_t*>(r.src),
+                                         reinterpret_cast<int32_t*>(r.dst), l.check, l.dst, l.bits, st);
     });
     seg->steps.back().ring_slot = l.slot1;
     seg->steps.back().ring_slot2 = l.slot2;

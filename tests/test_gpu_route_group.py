@@ -61,6 +61,15 @@ def test_grouping_gather_bit_exact(moe, orc, gpu_ctx, stream, pattern, T, E):
     _check_grouping_gather(moe, orc, gpu_ctx, stream, pattern, T, E)
 
 
+# One workgroup groups up to 80 tiles (8 or 40 counts held per thread): 409 tokens x 10 is 16
+# tiles, 410 is 17, 2048 is 80 and 2049 is 81.
+@pytest.mark.parametrize("E", [40, 512])
+@pytest.mark.parametrize("T", [409, 410, 2048, 2049])
+@pytest.mark.parametrize("pattern", ["mixed", "invalid_ids"])
+def test_grouping_one_workgroup_limits(moe, orc, gpu_ctx, stream, pattern, T, E):
+    _check_grouping_gather(moe, orc, gpu_ctx, stream, pattern, T, E)
+
+
 # The scan keeps up to 16 of its 256-entry tiles per thread in registers (512 tiles: N = 131072
 # entries); longer columns take its re-reading loop. 13107 tokens x 10 is 512 tiles, 16384 x 10
 # is 640.
