@@ -94,6 +94,28 @@ __device__ __forceinline__ uint32_t weight_fault(const uint8_t* w0, const uint8_
     return ((a | b) & 1u) ? 4u : 0u;
 }
 
+// Inclusive sum over the wave's 64 lanes by DPP (row shifts by 1, 2, 4, 8, then the last lane of a
+// 16-lane row into the next row and of the lower half into the upper): no LDS crossbar, whose six
+// exchanges cost about 130 cycles each. Every lane of the wave must be active.
+__device__ __forceinline__ uint32_t wave_scan(uint32_t v) {
+    v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x111, 0xF, 0xF, false));
+    v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x112, 0xF, 0xF, false));
+    v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x114, 0xF, 0xF, false));
+    v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x118, 0xF, 0xF, false));
+    v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x142, 0xA, 0xF, false));
+    v += uint32_t(__builtin_amdgcn_update_dpp(0, int(v), 0x143, 0xC, 0xF, false));
+    return v;
+}
+// Sum of the first `wave` of eight per-wave totals in LDS (all eight read at once).
+__device__ __forceinline__ uint32_t sum_before(const uint32_t* totals, uint32_t wave) {
+    uint32_t t[8], s = 0;
+#pragma unroll
+    for (uint32_t w = 0; w < 8u; ++w) t[w] = totals[w];
+#pragma unroll
+    for (uint32_t w = 0; w < 8u; ++w) s += w < wave ? t[w] : 0u;
+    return s;
+}
+
 // Called by a whole workgroup once each of its threads has issued the stores of what it read from
 // a pinned host slot (a store is issued after its data has arrived): tells the host, through one
 // pinned word (may be null), that the slot may be written again.

@@ -266,12 +266,7 @@ template <uint32_t NT>
 __device__ __forceinline__ uint32_t block_scan(uint32_t v, uint32_t* wave_tot, uint32_t& total) {
     constexpr uint32_t kWaves = NT / 64;
     const uint32_t lane = threadIdx.x & 63u, wave = threadIdx.x >> 6;
-    uint32_t inc = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-        const uint32_t o = __shfl_up(inc, off);
-        if (lane >= uint32_t(off)) inc += o;
-    }
+    const uint32_t inc = wave_scan(v);
     if (lane == 63u) wave_tot[wave] = inc;
     __syncthreads();
     uint32_t before = 0, all = 0;
@@ -479,14 +474,8 @@ __global__ __launch_bounds__(kScanThreads) void group_plan_kernel(uint32_t* __re
     const uint32_t own_hi = half == 0u ? nt_e | (count != 0u && !res ? 1u << 16 : 0u) : 0u;
     uint32_t lo = own_lo, hi = own_hi;
     if (half == 0u) {
-#pragma unroll
-        for (uint32_t off = 1; off < 64u; off <<= 1) {
-            const uint32_t a = __shfl_up(lo, off), b = __shfl_up(hi, off);
-            if (lane >= off) {
-                lo += a;
-                hi += b;
-            }
-        }
+        lo = wave_scan(lo);
+        hi = wave_scan(hi);
         if (lane == 63u) {
             s_lo[tid >> 6] = lo;
             s_hi[tid >> 6] = hi;

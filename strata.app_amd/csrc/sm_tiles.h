@@ -108,6 +108,17 @@ __device__ __forceinline__ void group_fields(const Plan* p, const int32_t* s_grp
     }
 }
 
+// The group holding item k of an enumeration: the last index lo with s_pref[lo] <= k (s_pref
+// ascends from s_pref[0] = 0; k < s_pref[512], uniform). Two LDS reads and a count each, where a
+// binary search is nine reads one after the other, at every item's start: with the scans by DPP
+// the gate/up stage of 512 experts went 197.3 -> 191.1 us at 2048 tokens (d 2048) and
+// 261.3 -> 253.3 at 1000 (d 2560), the stages of the smallest layer 10.6 + 10.4 -> 9.5 + 9.6.
+__device__ __forceinline__ uint32_t group_of(const uint32_t* s_pref, uint32_t k) {
+    const uint32_t lane = threadIdx.x & 63u;
+    const uint32_t seg = uint32_t(__builtin_popcountll(__ballot(s_pref[8u * lane] <= k))) - 1u;
+    return 8u * seg + uint32_t(__builtin_popcountll(__ballot(s_pref[8u * seg + (lane & 7u)] <= k) & 0xffull)) - 1u;
+}
+
 // Small-tile enumeration (512 threads, once per workgroup): groups below wide_min entries,
 // ceil(size / 64) tiles each; s_pref[gi] = tiles of the groups before gi, s_pref[512] = all.
 // Every group field is loaded without waiting for n_groups (thread gi < 512 reads inside the
@@ -117,9 +128,10 @@ __device__ __forceinline__ uint32_t scan_small_tiles(const RoutedGemm& g, uint32
                                                      int32_t* s_grp = nullptr) {
     const Plan* p = g.plan;
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    if (tid == 0) *s_flag = __hip_atomic_load(g.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t ng_raw = p->n_groups;
     const int32_t f = p->grp_start[tid], e = p->grp_start[tid + 1], ex = p->grp_e[tid];
+    // Behind the plan's loads, so that the first wave waits for all of them once.
+    if (tid == 0) *s_flag = __hip_atomic_load(g.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (s_grp != nullptr) stash_groups(s_grp, tid, f, e, ex);
     const uint32_t ng = ng_raw < 512u ? ng_raw : 512u;
     uint32_t n = 0;
@@ -130,15 +142,10 @@ __device__ __forceinline__ uint32_t scan_small_tiles(const RoutedGemm& g, uint32
             atomicOr(g.status, 2u);
         }
     }
-#pragma unroll
-    for (uint32_t off = 1; off < 64u; off <<= 1) {
-        const uint32_t y = __shfl_up(n, off);
-        if (lane >= off) n += y;
-    }
+    n = wave_scan(n);
     if (lane == 63u) s_wsum[wave] = n;
     __syncthreads();
-    uint32_t base = 0;
-    for (uint32_t w = 0; w < wave; ++w) base += s_wsum[w];
+    const uint32_t base = sum_before(s_wsum, wave);
     s_pref[tid + 1] = base + n;
     if (tid == 0) s_pref[0] = 0;
     __syncthreads();
@@ -154,12 +161,7 @@ __device__ __forceinline__ uint32_t staged_item_work(const RoutedGemm& g, const 
                                                      const int32_t* s_grp) {
     const Plan* p = g.plan;
     const uint32_t k = item / n_chunks, chunk = item - k * n_chunks;
-    uint32_t lo = 0, hi = 512;
-    while (hi - lo > 1u) {
-        const uint32_t mid = (lo + hi) >> 1;
-        if (s_pref[mid] <= k) lo = mid;
-        else hi = mid;
-    }
+    const uint32_t lo = group_of(s_pref, k);
     uint32_t f, e, ex;
     group_fields(p, s_grp, lo, f, e, ex);
     t.nt_begin = chunk * npi;

@@ -253,9 +253,10 @@ __device__ __forceinline__ uint32_t scan_wide_units(const RoutedGemm& g, uint32_
                                                     int32_t* s_grp = nullptr) {
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const Plan* p = g.plan;
-    if (tid == 0) *s_flag = __hip_atomic_load(g.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const uint32_t ng_raw = p->n_groups;
     const int32_t f = p->grp_start[tid], e = p->grp_start[tid + 1], ex = p->grp_e[tid];
+    // Behind the plan's loads, so that the first wave waits for all of them once.
+    if (tid == 0) *s_flag = __hip_atomic_load(g.status, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     if (s_grp != nullptr) stash_groups(s_grp, tid, f, e, ex);
     const uint32_t ng = ng_raw < 512u ? ng_raw : 512u;
     uint32_t units = 0, tiles = 0;
@@ -267,25 +268,13 @@ __device__ __forceinline__ uint32_t scan_wide_units(const RoutedGemm& g, uint32_
             atomicOr(g.status, 2u);
         }
     }
-    uint32_t incl = units, incl_t = tiles;
-#pragma unroll
-    for (uint32_t off = 1; off < 64u; off <<= 1) {
-        const uint32_t y = __shfl_up(incl, off), yt = __shfl_up(incl_t, off);
-        if (lane >= off) {
-            incl += y;
-            incl_t += yt;
-        }
-    }
+    const uint32_t incl = wave_scan(units), incl_t = wave_scan(tiles);
     if (lane == 63u) {
         s_wsum[wave] = incl;
         if (s_tiles != nullptr) s_tsum[wave] = incl_t;
     }
     __syncthreads();
-    uint32_t base = 0, base_t = 0;
-    for (uint32_t w = 0; w < wave; ++w) {
-        base += s_wsum[w];
-        if (s_tiles != nullptr) base_t += s_tsum[w];
-    }
+    const uint32_t base = sum_before(s_wsum, wave), base_t = s_tiles != nullptr ? sum_before(s_tsum, wave) : 0u;
     s_pref[tid + 1] = base + incl;
     if (tid == 0) s_pref[0] = 0;
     if (s_tiles != nullptr) {
@@ -350,12 +339,7 @@ __device__ __forceinline__ void wide_items(const RoutedGemm& g, const uint8_t* d
             u.a1 = u.a0 + kUnitRows < g.n_entries ? u.a0 + kUnitRows : g.n_entries;
             u.ex = 0;
         } else {
-            uint32_t lo_g = 0, hi_g = 512;
-            while (hi_g - lo_g > 1u) {
-                const uint32_t mid = (lo_g + hi_g) >> 1;
-                if (s_pref[mid] <= uidx) lo_g = mid;
-                else hi_g = mid;
-            }
+            const uint32_t lo_g = group_of(s_pref, uidx);
             uint32_t f, e, ex;
             group_fields(p, s_grp, lo_g, f, e, ex);
             const uint32_t usz = unit_rows(e - f);
