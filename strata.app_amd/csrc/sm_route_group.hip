@@ -592,15 +592,32 @@ __global__ __launch_bounds__(256) void group_scatter_kernel(const int32_t* __res
 // Expert-stage validation (prefill_moe.metal:603-733): status is cleared, then bit 1 set
 // when the plan header, the tile chain, or the destination permutation is inconsistent.
 // ---------------------------------------------------------------------------------------
-// The header and per-group checks run one group per thread; the tile-count sum is a block
-// reduction, so the whole plan is checked in a few dependent memory round trips.
+// The header and per-group checks run from registers and LDS after one round trip for the whole
+// plan; the tile list is a second one. (Header, groups and tile chain read one after the other
+// behind the address tables made the checked gather 11.2 us by events instead of 8.9 at 100
+// tokens.)
 // The whole check runs in one workgroup of NT threads; `reset_status` clears the status
 // words first (a full layer's gather leaves that to the grouping, see GroupPrep).
 template <uint32_t NT>
 __device__ __forceinline__ void check_plan(const PlanCheck& c, bool reset_status) {
-    __shared__ uint32_t s_header_ok, s_groups_ok, s_wave_tiles[NT / 64];
+    __shared__ uint32_t s_groups_ok, s_wave_tiles[NT / 64];
+    __shared__ int32_t s_start[513], s_ex[512];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
-    if (tid < c.n_counters) c.counters[tid] = 0u;
+    const Plan* p = c.plan;
+    const uint32_t N = c.n_entries, E = c.n_experts;
+    // The plan's fields go out together (thread g reads inside the plan's arrays whatever n_groups
+    // holds), ahead of the address tables: loads return in order, and the tables come from pinned
+    // host memory, so the checks run while they travel.
+    const uint32_t ng = p->n_groups, nt = p->n_tiles, n_entries = p->n_entries, bad = p->bad;
+    constexpr uint32_t kGroups = 512u / NT;
+    int32_t first[kGroups], end[kGroups], ex[kGroups];
+#pragma unroll
+    for (uint32_t j = 0; j < kGroups; ++j) {
+        first[j] = p->grp_start[tid + NT * j];
+        end[j] = p->grp_start[tid + NT * j + 1u];
+        ex[j] = p->grp_e[tid + NT * j];
+    }
+    __asm__ volatile("" ::: "memory");
     // Address snapshots: every load of a thread is issued before its stores, so the reads
     // of pinned host memory cost one round trip (tables are at most 3 x 512 words).
     constexpr int kPer = 1536 / NT;
@@ -611,15 +628,8 @@ __device__ __forceinline__ void check_plan(const PlanCheck& c, bool reset_status
         v1[j] = c.snap_src != nullptr && i < c.snap_words ? c.snap_src[i] : 0u;
         v2[j] = c.snap_src2 != nullptr && i < c.snap_words2 ? c.snap_src2[i] : 0u;
     }
-#pragma unroll
-    for (int j = 0; j < kPer; ++j) {
-        const uint32_t i = tid + NT * j;
-        if (c.snap_src != nullptr && i < c.snap_words) c.snap_dst[i] = v1[j];
-        if (c.snap_src2 != nullptr && i < c.snap_words2) c.snap_dst2[i] = v2[j];
-    }
-    const Plan* p = c.plan;
-    const uint32_t N = c.n_entries, E = c.n_experts;
-    const uint32_t ng = p->n_groups, nt = p->n_tiles;
+    __asm__ volatile("" ::: "memory");
+    if (tid < c.n_counters) c.counters[tid] = 0u;
     auto fail = [&]() {
         atomicOr(c.status, 2u);
         if (c.status2 != nullptr) atomicOr(c.status2, 2u);
@@ -630,55 +640,64 @@ __device__ __forceinline__ void check_plan(const PlanCheck& c, bool reset_status
             if (c.status2 != nullptr) *c.status2 = 0u;
         }
         s_groups_ok = 1u;
-        s_header_ok = (p->bad == 0u && ng != 0u && ng <= E && ng <= 512u && p->n_entries == N &&
-                       nt <= c.tile_capacity && nt <= p->n_entries && p->grp_start[0] == 0 &&
-                       p->grp_start[ng] == int32_t(N))
-                          ? 1u : 0u;
-    }
-    report_read(c.done, c.done_value);  // (its barrier also shows s_header_ok)
-    if (!s_header_ok) {
-        if (tid == 0) fail();
-        return;
-    }
-    // Group g: non-empty, inside [0, N), expert in range and strictly ascending.
-    uint32_t my_tiles = 0;
-    for (uint32_t g = tid; g < ng; g += NT) {
-        const int32_t first = p->grp_start[g], end = p->grp_start[g + 1], ex = p->grp_e[g];
-        bool ok = end > first && uint32_t(end) <= N && ex >= 0 && uint32_t(ex) < E;
-        if (g != 0u) ok = ok && ex > p->grp_e[g - 1];
-        if (!ok) s_groups_ok = 0u;
-        else my_tiles += (uint32_t(end - first) + kExpertTile - 1) / kExpertTile;
     }
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) my_tiles += __shfl_xor(my_tiles, off);
-    if (lane == 0) s_wave_tiles[wave] = my_tiles;
+    for (uint32_t j = 0; j < kGroups; ++j) {
+        s_start[tid + NT * j] = first[j];
+        s_ex[tid + NT * j] = ex[j];
+    }
+    if (tid == NT - 1u) s_start[512] = end[kGroups - 1u];
+    __syncthreads();
+    const bool header_ok = bad == 0u && ng != 0u && ng <= E && ng <= 512u && n_entries == N && nt <= c.tile_capacity &&
+                           nt <= n_entries && s_start[0] == 0 && s_start[ng <= 512u ? ng : 0u] == int32_t(N);
+    // Group g: non-empty, inside [0, N), expert in range and strictly ascending.
+    uint32_t my_tiles = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kGroups; ++j) {
+        const uint32_t g = tid + NT * j;
+        if (!header_ok || g >= ng) continue;
+        bool ok = end[j] > first[j] && uint32_t(end[j]) <= N && ex[j] >= 0 && uint32_t(ex[j]) < E;
+        if (g != 0u) ok = ok && ex[j] > s_ex[g - 1u];
+        if (!ok) s_groups_ok = 0u;
+        else my_tiles += (uint32_t(end[j] - first[j]) + kExpertTile - 1) / kExpertTile;
+    }
+    my_tiles = wave_scan(my_tiles);
+    if (lane == 63u) s_wave_tiles[wave] = my_tiles;
     __syncthreads();
     uint32_t expected = 0;
+#pragma unroll
     for (uint32_t w = 0; w < NT / 64; ++w) expected += s_wave_tiles[w];
-    if (!s_groups_ok || expected != nt) {
+    if (!header_ok || !s_groups_ok || expected != nt) {
         if (tid == 0) fail();
-        return;
-    }
-    const uint32_t* tiles = c.tiles;
-    for (uint32_t i = tid; i < nt; i += NT) {
-        const uint32_t tg = tiles[2 * i], ty = tiles[2 * i + 1];
-        bool ok = tg < ng;
-        if (ok) {
-            const uint32_t first = uint32_t(p->grp_start[tg]), end = uint32_t(p->grp_start[tg + 1]);
-            ok = ty >= first && ty < end && (ty - first) % kExpertTile == 0u;
-            if (i == 0u) {
-                ok = ok && tg == 0u && ty == 0u;
-            } else {
-                const uint32_t pg = tiles[2 * (i - 1)], py = tiles[2 * (i - 1) + 1];
-                if (pg >= ng) ok = false;
-                else if (pg == tg) ok = ok && ty == py + kExpertTile;
-                else if (pg + 1u == tg) ok = ok && py + kExpertTile >= uint32_t(p->grp_start[pg + 1]) && ty == first;
-                else ok = false;
+    } else {
+        const uint32_t* tiles = c.tiles;
+        for (uint32_t i = tid; i < nt; i += NT) {
+            const uint32_t tg = tiles[2 * i], ty = tiles[2 * i + 1];
+            const uint32_t pg = i != 0u ? tiles[2 * (i - 1)] : 0u, py = i != 0u ? tiles[2 * (i - 1) + 1] : 0u;
+            bool ok = tg < ng;
+            if (ok) {
+                const uint32_t start = uint32_t(s_start[tg]), stop = uint32_t(s_start[tg + 1]);
+                ok = ty >= start && ty < stop && (ty - start) % kExpertTile == 0u;
+                if (i == 0u) {
+                    ok = ok && tg == 0u && ty == 0u;
+                } else {
+                    if (pg >= ng) ok = false;
+                    else if (pg == tg) ok = ok && ty == py + kExpertTile;
+                    else if (pg + 1u == tg) ok = ok && py + kExpertTile >= uint32_t(s_start[pg + 1]) && ty == start;
+                    else ok = false;
+                }
+                if (i + 1u == nt) ok = ok && tg + 1u == ng && ty + kExpertTile >= stop;
             }
-            if (i + 1u == nt) ok = ok && tg + 1u == ng && ty + kExpertTile >= end;
+            if (!ok) fail();
         }
-        if (!ok) fail();
     }
+#pragma unroll
+    for (int j = 0; j < kPer; ++j) {
+        const uint32_t i = tid + NT * j;
+        if (c.snap_src != nullptr && i < c.snap_words) c.snap_dst[i] = v1[j];
+        if (c.snap_src2 != nullptr && i < c.snap_words2) c.snap_dst2[i] = v2[j];
+    }
+    report_read(c.done, c.done_value);
 }
 
 __global__ __launch_bounds__(512) void plan_validate_kernel(PlanCheck c) {
@@ -744,7 +763,10 @@ __global__ __launch_bounds__(256) void gather_kernel(const u32x4* __restrict__ x
     load_batch(t0);
     const uint64_t entry = uint64_t(i0) + tid;
     const int32_t id = entry < N ? ids[entry] : -1;  // issued before the plan reads
-    for (uint32_t e = tid; e < E; e += 256u) s_base[e] = hist[uint64_t(tile) * E + e];
+    // (E <= 512: two cursors per thread, loaded with the rest and stored behind all of it.)
+    uint32_t cursor[2];
+#pragma unroll
+    for (uint32_t q = 0; q < 2u; ++q) cursor[q] = hist[uint64_t(tile) * E + (tid + 256u * q < E ? tid + 256u * q : E - 1u)];
     const uint32_t ng = plan->n_groups, p_entries = plan->n_entries, p_bad = plan->bad;
     // CHECK: this workgroup's share of the tile's destinations, loaded with the other first
     // loads and marked after the copies (a returning atomic would hold the copies behind its
@@ -767,7 +789,8 @@ __global__ __launch_bounds__(256) void gather_kernel(const u32x4* __restrict__ x
             if (atomicOr(&bits[dv / 32u], mask) & mask) atomicOr(c.status2, 2u);
         }
     };
-    for (uint32_t k = tid; k < 4u * 512u; k += 256u) (&wcnt[0][0])[k] = 0u;
+#pragma unroll
+    for (uint32_t k = 0; k < 8u; ++k) (&wcnt[0][0])[tid + 256u * k] = 0u;
     // The entry's slot, as group_scatter_kernel computes it.
     const bool valid = id >= 0 && uint32_t(id) < E;
     const uint32_t key = valid ? uint32_t(id) : 1023u;
@@ -782,6 +805,8 @@ __global__ __launch_bounds__(256) void gather_kernel(const u32x4* __restrict__ x
     const uint64_t gt = lane == 63u ? 0ull : (~0ull << (lane + 1u));
     // The plan header's second look-up travels while the slots are computed.
     const int32_t sorted_signed = plan->grp_start[ng <= 512u ? ng : 0u];
+#pragma unroll
+    for (uint32_t q = 0; q < 2u; ++q) s_base[tid + 256u * q] = cursor[q];
     __syncthreads();
     if (valid && (match & gt) == 0ull) wcnt[wave][id] = rank + 1u;
     __syncthreads();
