@@ -26,14 +26,24 @@ namespace {
 // in flight. The ring stays within 96 KB so that a workgroup of the shared expert's GEMM,
 // which runs beside the router on the second stream, still fits on the same CU. Within a
 // wave the k-steps keep the order of a plain loop over its columns.
+// G = 2 (up to kRouterPairRows tokens, 32-token tiles): the stages go in pairs, one barrier and one
+// wait for operands per pair, through a ring of three pairs (120 KB, four stages in flight instead
+// of three). With so few tokens a workgroup's serial chain over d is the launch, and its CU has
+// room. The sums keep their order, so the logits are the same bits. Routing alone: 100 tokens
+// 26.4 -> 25.4 us (512 experts, d 2048), 500 tokens 38.9 -> 36.8 (256, 4096), 800 tokens 32.8 ->
+// 31.7; layers: 513 tokens of 128 experts 190.5 -> 186.9, 500 of 512 experts 358.9 -> 353.2, 800
+// 378.6 -> 377.3 and without a shared expert the same. At 2000 tokens of 128 experts the ring
+// shuts the shared expert's workgroups out of more CUs and the layer went 394 -> 399.5 us.
 // ---------------------------------------------------------------------------------------
 constexpr int kRouterCols = 64;
 constexpr int kRouterThreads = 512;
+constexpr uint32_t kRouterPairRows = 800;  // stages in pairs up to this many tokens
 
-template <int ROWS>
+template <int ROWS, int G>
 struct RouterStage {
     static constexpr int KS = 64;                      // reduction columns per stage
-    static constexpr int NST = ROWS == 128 ? 3 : 4;    // ring slots (NST - 1 stages in flight)
+    static constexpr int NGR = ROWS == 128 || G == 2 ? 3 : 4;  // ring slots of G stages (NGR - 1 in flight)
+    static constexpr int NST = NGR * G;
     static constexpr int CPR = KS / 8;                 // 16-byte activation chunks per row
     static constexpr int RPI = 64 / CPR;               // activation rows per copy instruction
     static constexpr int NA = ROWS / (4 * RPI);        // activation copies per copying wave and stage
@@ -43,7 +53,8 @@ struct RouterStage {
     static constexpr int A_BYTES = ROWS * KS * 2;
     static constexpr int BYTES = A_BYTES + kRouterCols * KS * 4;
     static_assert(NA * 4 * RPI == ROWS && NW * WPI == 16, "copy map covers the stage");
-    static_assert(NST * BYTES <= 96 * 1024, "LDS ring leaves room for a co-resident workgroup");
+    static_assert(G == 2 || NST * BYTES <= 96 * 1024, "LDS ring leaves room for a co-resident workgroup");
+    static_assert(NST * BYTES <= 160 * 1024, "LDS ring fits a CU");
     // The second k-half's partial sums (ROWS / 16 blocks x 4 values x head and tail, for
     // 256 lanes) pass through the ring after the last stage.
     static_assert(ROWS / 16 * 8 * 256 * 4 <= NST * BYTES, "partial sums fit the ring");
@@ -53,14 +64,14 @@ struct RouterStage {
 // vmcnt in bits 3:0 and 15:14; expcnt and lgkmcnt left at their no-wait maxima).
 constexpr int vmcnt_imm(int n) { return (n & 15) | ((n >> 4) << 14) | (7 << 4) | (15 << 8); }
 
-template <int ROWS>
+template <int ROWS, int G>
 __global__ __launch_bounds__(kRouterThreads) void router_gemm_kernel(const _Float16* __restrict__ x,
                                                                     const float* __restrict__ w,
                                                                     const float* __restrict__ bias,
                                                                     float* __restrict__ logits,
                                                                     uint32_t rows, uint32_t d, uint32_t E,
                                                                     RouterPrep prep) {
-    using S = RouterStage<ROWS>;
+    using S = RouterStage<ROWS, G>;
     constexpr int RB = ROWS / 16;  // 16-row MFMA blocks
     typedef float f2v __attribute__((ext_vector_type(2)));
     typedef _Float16 h2v __attribute__((ext_vector_type(2)));
@@ -121,56 +132,68 @@ __global__ __launch_bounds__(kRouterThreads) void router_gemm_kernel(const _Floa
     float4v acc_hi[RB], acc_lo[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; ++rb) { acc_hi[rb] = float4v{0, 0, 0, 0}; acc_lo[rb] = float4v{0, 0, 0, 0}; }
-    const uint32_t n_st = d / S::KS;
+    const uint32_t n_gr = d / (S::KS * G);
+    auto issue_group = [&](uint32_t gr) {
+#pragma unroll
+        for (uint32_t z = 0; z < uint32_t(G); ++z) issue(gr * G + z, gr % S::NGR * G + z);
+    };
     if (copier) {
 #pragma unroll
-        for (int i = 0; i < S::NST - 1; ++i)
-            if (uint32_t(i) < n_st) issue(i, i);
+        for (int i = 0; i < S::NGR - 1; ++i)
+            if (uint32_t(i) < n_gr) issue_group(i);
     }
     const uint32_t wrow = 16u * wave + n;  // this lane's expert row in the weight slab
     const uint32_t c0 = 8u * kh + 2u * g;   // lane group g holds columns 8g .. 8g + 7 of the k-step
-    for (uint32_t st = 0; st < n_st; ++st) {
-        // Stage st's copies (of every copying wave, hence the barrier); stage st + 1 may stay
+    for (uint32_t gr = 0; gr < n_gr; ++gr) {
+        // Group gr's copies (of every copying wave, hence the barrier); the later ones may stay
         // in flight. A bare s_barrier: __syncthreads() would add a workgroup release that
-        // waits for every copy in flight. A copying wave's stage-st copies are complete after
+        // waits for every copy in flight. A copying wave's copies of the group are complete after
         // the wait, and the slot refilled below was last read in the previous iteration, whose
         // LDS reads every wave consumed before reaching this barrier.
         if (copier) {
-            const uint32_t later = n_st - 1u - st;  // stages issued after st (at most NST - 2)
-            if (S::NST == 4 && later >= 2u) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * (S::NA + S::NW)));
-            else if (later >= 1u) __builtin_amdgcn_s_waitcnt(vmcnt_imm(S::NA + S::NW));
+            const uint32_t later = n_gr - 1u - gr;  // groups issued after gr (at most NGR - 2)
+            if (S::NGR == 4 && later >= 2u) __builtin_amdgcn_s_waitcnt(vmcnt_imm(2 * G * (S::NA + S::NW)));
+            else if (later >= 1u) __builtin_amdgcn_s_waitcnt(vmcnt_imm(G * (S::NA + S::NW)));
             else __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));
         }
         __builtin_amdgcn_s_barrier();
-        if (copier && st + S::NST - 1 < n_st) issue(st + S::NST - 1, (st + S::NST - 1) % S::NST);
-        const uint8_t* base = ring + (st % S::NST) * S::BYTES;
-        const uint8_t* wb = base + S::A_BYTES + wrow * (S::KS * 4);
-        // Every operand read of the k-step first, then the split, so one wait covers them.
-        const float4v w0 = *reinterpret_cast<const float4v*>(wb + 16u * (c0 ^ uint32_t(n)));
-        const float4v w1 = *reinterpret_cast<const float4v*>(wb + 16u * ((c0 + 1u) ^ uint32_t(n)));
-        half8 a[RB];
+        if (copier && gr + S::NGR - 1 < n_gr) issue_group(gr + S::NGR - 1);
+        // Every operand read of the group's k-steps first, then the splits, so one wait covers them.
+        float4v w0[G], w1[G];
+        half8 a[G][RB];
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            const uint32_t r = 16u * rb + n;
-            const uint32_t pos = (4u * kh + g) ^ (r % S::CPR);
-            a[rb] = *reinterpret_cast<const half8*>(base + r * (S::KS * 2) + 16u * pos);
+        for (int z = 0; z < G; ++z) {
+            const uint8_t* base = ring + (gr % S::NGR * G + z) * S::BYTES;
+            const uint8_t* wb = base + S::A_BYTES + wrow * (S::KS * 4);
+            w0[z] = *reinterpret_cast<const float4v*>(wb + 16u * (c0 ^ uint32_t(n)));
+            w1[z] = *reinterpret_cast<const float4v*>(wb + 16u * ((c0 + 1u) ^ uint32_t(n)));
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                const uint32_t r = 16u * rb + n;
+                const uint32_t pos = (4u * kh + g) ^ (r % S::CPR);
+                a[z][rb] = *reinterpret_cast<const half8*>(base + r * (S::KS * 2) + 16u * pos);
+            }
         }
         __builtin_amdgcn_sched_barrier(0);
-        half8 bh, bl;
+        if (G > 1) __builtin_amdgcn_s_waitcnt(15 | (3 << 14) | (7 << 4));  // lgkmcnt(0): the group's reads are done
 #pragma unroll
-        for (int i = 0; i < 8; i += 2) {
-            const f2v wv = i < 4 ? f2v{w0[i], w0[i + 1]} : f2v{w1[i - 4], w1[i - 3]};
-            const h2v hp = __builtin_convertvector(wv, h2v);                                     // head, RNE
-            const h2v lp = __builtin_convertvector((wv - __builtin_convertvector(hp, f2v)) * 2048.0f, h2v);  // tail
-            bh[i] = hp.x;
-            bh[i + 1] = hp.y;
-            bl[i] = lp.x;
-            bl[i + 1] = lp.y;
-        }
+        for (int z = 0; z < G; ++z) {
+            half8 bh, bl;
 #pragma unroll
-        for (int rb = 0; rb < RB; ++rb) {
-            acc_hi[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[rb], bh, acc_hi[rb], 0, 0, 0);
-            acc_lo[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[rb], bl, acc_lo[rb], 0, 0, 0);
+            for (int i = 0; i < 8; i += 2) {
+                const f2v wv = i < 4 ? f2v{w0[z][i], w0[z][i + 1]} : f2v{w1[z][i - 4], w1[z][i - 3]};
+                const h2v hp = __builtin_convertvector(wv, h2v);                                     // head, RNE
+                const h2v lp = __builtin_convertvector((wv - __builtin_convertvector(hp, f2v)) * 2048.0f, h2v);  // tail
+                bh[i] = hp.x;
+                bh[i + 1] = hp.y;
+                bl[i] = lp.x;
+                bl[i + 1] = lp.y;
+            }
+#pragma unroll
+            for (int rb = 0; rb < RB; ++rb) {
+                acc_hi[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[z][rb], bh, acc_hi[rb], 0, 0, 0);
+                acc_lo[rb] = __builtin_amdgcn_mfma_f32_16x16x32_f16(a[z][rb], bl, acc_lo[rb], 0, 0, 0);
+            }
         }
     }
     // The second k-half hands its partial sums to the first through the ring (every wave's
@@ -878,11 +901,13 @@ hipError_t launch_router_gemm(const _Float16* x, const float* w, const float* bi
     const uint32_t ecols = (E + kRouterCols - 1) / kRouterCols;
     auto blocks = [&](uint32_t r) { return ((rows + r - 1) / r) * ecols; };
     if (blocks(128) >= 256u) {
-        router_gemm_kernel<128><<<dim3((rows + 127) / 128, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
+        router_gemm_kernel<128, 1><<<dim3((rows + 127) / 128, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
     } else if (blocks(64) >= 256u) {
-        router_gemm_kernel<64><<<dim3((rows + 63) / 64, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
+        router_gemm_kernel<64, 1><<<dim3((rows + 63) / 64, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
+    } else if (rows <= kRouterPairRows && d % 128u == 0u) {
+        router_gemm_kernel<32, 2><<<dim3((rows + 31) / 32, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
     } else {
-        router_gemm_kernel<32><<<dim3((rows + 31) / 32, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
+        router_gemm_kernel<32, 1><<<dim3((rows + 31) / 32, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
     }
     return hipGetLastError();
 }

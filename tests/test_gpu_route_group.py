@@ -151,3 +151,18 @@ def test_route_gather_composition(moe, layer, orc, gpu_ctx, stream, cfg_index):
     assert np.array_equal(gu.host(ws.dst, np.int32)[:n_valid], g["dst"][:n_valid])
     xs = gu.host(ws.xs, np.uint16).reshape(T * K, d)
     assert np.array_equal(xs[:n_valid], orc.gather(inp.x[:T], g["src"], n_valid))
+
+
+@pytest.mark.parametrize("T,E,d", [(1, 16, 256), (33, 65, 512), (100, 512, 768), (800, 256, 1280), (801, 256, 1280)])
+def test_router_few_tiles(moe, layer, orc, gpu_ctx, stream, T, E, d):
+    """Router logits with 2 to 10 stage pairs, ragged token and expert tiles, and on both sides of
+    the token count up to which stages run in pairs (800)."""
+    print(f"case router T={T} E={E} d={d}", flush=True)
+    cfg = layer.LayerConfig("router_few", T, d, E, 4, 128, 0, moe.Q8_0, moe.Q8_0, moe.F16, seed=95)
+    inp = layer.make_inputs(cfg, with_experts=False)
+    ws = layer.LayerWorkspace(gpu_ctx, cfg, inp)
+    rg = ws.route_gather_buffers()
+    gu.run(gpu_ctx, stream, lambda s: s.encode_prefill_moe_full_mode_route_gather(cfg.shape(), rg))
+    logits = gu.host(ws.logits, np.float32).reshape(T, E)
+    mag = np.abs(inp.x[:T].view(np.float16).astype(np.float64)) @ np.abs(inp.w_router.astype(np.float64)).T
+    assert (np.abs(logits - orc.router_ref(inp.x[:T], inp.w_router)) <= 2.0 ** -20 * mag + 1e-7).all(), "router logits"
