@@ -467,15 +467,34 @@ bool ring_reached(const sm_context* ctx, uint32_t slot) {
     return true;
 }
 
-// Waits until the launch that reads a pending slot has read it. After a second the whole device
-// is waited for instead, so that a device error ends the wait (false).
+// Whether the device still answers: asked of the context's own side stream, which no capture
+// includes, without waiting for anything.
+bool device_answers(const sm_context* ctx) {
+    const hipError_t e = hipStreamQuery(ctx->side);
+    // "Not ready" is no error: it must not be what the thread's next launch reports.
+    if (e == hipErrorNotReady && hipPeekAtLastError() == hipErrorNotReady) (void)hipGetLastError();
+    return e == hipSuccess || e == hipErrorNotReady;
+}
+
+// Waits, however long it takes, until the launch that reads a pending slot has read it: the poll
+// is closest in the first 200 us and sleeps from then on (the caller is 32 layers ahead of the
+// GPU). Nothing else on the device is waited for; false only if the device reports an error.
+// Called without ring_mu: a waiting encode holds up no other thread's claims and commits.
 bool wait_ring(const sm_context* ctx, uint32_t slot) {
-    const auto t0 = std::chrono::steady_clock::now();
-    for (uint32_t n = 1; !ring_reached(ctx, slot); ++n) {
-        if (n % 1024u != 0u) continue;
-        std::this_thread::yield();
-        if (std::chrono::steady_clock::now() - t0 > std::chrono::seconds(1))
-            return hipSetDevice(ctx->device) == hipSuccess && hipDeviceSynchronize() == hipSuccess && ring_reached(ctx, slot);
+    using clock = std::chrono::steady_clock;
+    const auto t0 = clock::now();
+    auto asked = t0;
+    while (!ring_reached(ctx, slot)) {
+        const auto now = clock::now();
+        if (now - t0 < std::chrono::microseconds(200)) {
+            std::this_thread::yield();
+            continue;
+        }
+        if (now - asked > std::chrono::milliseconds(100)) {
+            if (!device_answers(ctx)) return ring_reached(ctx, slot);
+            asked = now;
+        }
+        std::this_thread::sleep_for(std::chrono::microseconds(20));
     }
     return true;
 }
@@ -494,19 +513,29 @@ RingMark ring_mark(sm_context* ctx, int slot) {
 // -3 when waiting for a slot's previous copy failed.
 int claim_ring_slot(sm_context* ctx, const std::vector<uint64_t>& table) {
     if (ctx->ring == nullptr) return -1;
-    std::lock_guard<std::mutex> lk(ctx->ring_mu);
-    for (uint32_t tries = 0; tries < sm_context::kRingSlots; ++tries) {
-        const uint32_t slot = ctx->ring_next++ % sm_context::kRingSlots;
-        if (ctx->ring_claimed[slot]) continue;
-        if (ctx->ring_pending[slot]) {
-            if (!wait_ring(ctx, slot)) return -3;
-            ctx->ring_pending[slot] = false;
+    int slot = -1;
+    bool pending = false;
+    {
+        std::lock_guard<std::mutex> lk(ctx->ring_mu);
+        for (uint32_t tries = 0; slot < 0 && tries < sm_context::kRingSlots; ++tries) {
+            const uint32_t s = ctx->ring_next++ % sm_context::kRingSlots;
+            if (!ctx->ring_claimed[s]) slot = int(s);
         }
-        ctx->ring_claimed[slot] = true;
-        std::memcpy(ctx->ring + uint64_t(slot) * sm_context::kSlotWords, table.data(), table.size() * 8);
-        return int(slot);
+        if (slot < 0) return -2;
+        ctx->ring_claimed[slot] = true;  // from here on the slot is this thread's
+        pending = ctx->ring_pending[slot];
     }
-    return -2;
+    if (pending) {
+        const bool reached = wait_ring(ctx, uint32_t(slot));
+        std::lock_guard<std::mutex> lk(ctx->ring_mu);
+        if (!reached) {
+            ctx->ring_claimed[slot] = false;  // still pending
+            return -3;
+        }
+        ctx->ring_pending[slot] = false;
+    }
+    std::memcpy(ctx->ring + uint64_t(slot) * sm_context::kSlotWords, table.data(), table.size() * 8);
+    return slot;
 }
 
 void release_ring_slots(sm_segment* seg) {

@@ -94,3 +94,90 @@ def test_ring_reuse_through_stage_entry_points(moe, layer, gpu_ctx, stream):
     torch.cuda.synchronize()
     for b, w in zip(outs, want):
         assert np.array_equal(gu.host(b, np.uint32), w)
+
+
+def _spin(stream, ms, rate):
+    """Keeps `stream` busy for about `ms` with one workgroup; the event behind it."""
+    import torch
+    with torch.cuda.stream(stream):
+        torch.cuda._sleep(int(ms * rate))
+        ev = torch.cuda.Event()
+        ev.record()
+    return ev
+
+
+def _spin_rate():
+    """Cycles of torch.cuda._sleep per millisecond."""
+    import torch
+    torch.cuda._sleep(1000)
+    a, b = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+    a.record()
+    torch.cuda._sleep(10_000_000)
+    b.record()
+    torch.cuda.synchronize()
+    return 10_000_000 / a.elapsed_time(b)
+
+
+def _independent_streams(rate):
+    """Two streams that run beside each other (several streams may share one hardware queue)."""
+    import torch
+    first = torch.cuda.Stream()
+    for _ in range(8):
+        other = torch.cuda.Stream()
+        late, early = _spin(other, 100, rate), _spin(first, 1, rate)
+        early.synchronize()
+        beside = not late.query()
+        torch.cuda.synchronize()
+        if beside:
+            return first, other
+    pytest.skip("no two streams with hardware queues of their own")
+
+
+def test_full_ring_waits_for_its_own_launches_only(moe, layer):
+    """64 slots read by layers queued behind 1.5 s of other work: the next encode waits for the
+    first of them, and for nothing else. Work on an unrelated stream is still running when it
+    returns, and another thread's commit on the context is not held up while it waits."""
+    import threading
+    import time
+
+    import torch
+    print("case ring full behind other work", flush=True)
+    ctx = moe.Context(0)
+    ws = [layer.DecodeWorkspace(ctx, c, layer.make_inputs(c)) for c in (_decode(layer, moe, 0xC0C2A),
+                                                                       _decode(layer, moe, 0xC0C2B))]
+    main = torch.cuda.current_stream().cuda_stream
+    want = []
+    for w in ws:
+        w.run(main)
+        torch.cuda.synchronize()
+        want.append(_out(w))
+        w.out.tensor.fill_(7.0)
+    rate = _spin_rate()
+    a, b = _independent_streams(rate)
+    late = _spin(b, 4000, rate)
+    gate = _spin(a, 1500, rate)
+    ready = ctx.segment()  # encoded ahead: two of the 64 slots, not yet committed
+    ok, err = ws[1].encode(ready)
+    assert ok, err
+    for _ in range(31):
+        ws[0].run(a.cuda_stream)
+    assert not gate.query()
+    done = []
+
+    def next_layer():
+        ws[0].run(a.cuda_stream)
+        done.append((gate.query(), late.query()))
+
+    t = threading.Thread(target=next_layer)
+    t.start()
+    time.sleep(0.2)
+    assert t.is_alive() and not gate.query(), "the encode did not have to wait"
+    ready.commit(a.cuda_stream)
+    held_up = gate.query() or not t.is_alive()
+    t.join()
+    torch.cuda.synchronize()
+    assert not held_up, "a commit waited for another thread's encode"
+    assert done == [(True, False)], "the encode waited for an unrelated stream"
+    for w, o in zip(ws, want):
+        assert w.read_status() == 0
+        assert np.array_equal(_out(w).view(np.uint32), o.view(np.uint32))
