@@ -46,8 +46,11 @@ struct sm_context {
     // it. A step that reads two slots reports in its first slot's row for both. The values of a
     // row only grow: a slot's next use is claimed after its last one was waited for, and the
     // launches of one use run in order on the commit's own stream.
-    struct RingWait { uint32_t slot, value, words; };
+    // by_event: the step failed, so it may never report, and the slot's own event (made then) is
+    // waited for instead.
+    struct RingWait { uint32_t slot, value, words; bool by_event; };
     RingWait ring_wait[kRingSlots] = {};
+    hipEvent_t ring_ev[kRingSlots] = {};
     bool ring_pending[kRingSlots] = {};
     bool ring_claimed[kRingSlots] = {};  // filled by an encode whose segment is not committed yet
     uint32_t ring_next = 0;
@@ -481,6 +484,7 @@ bool device_answers(const sm_context* ctx) {
 // GPU). Nothing else on the device is waited for; false only if the device reports an error.
 // Called without ring_mu: a waiting encode holds up no other thread's claims and commits.
 bool wait_ring(const sm_context* ctx, uint32_t slot) {
+    if (ctx->ring_wait[slot].by_event) return hipEventSynchronize(ctx->ring_ev[slot]) == hipSuccess;
     using clock = std::chrono::steady_clock;
     const auto t0 = clock::now();
     auto asked = t0;
@@ -536,6 +540,18 @@ int claim_ring_slot(sm_context* ctx, const std::vector<uint64_t>& table) {
     }
     std::memcpy(ctx->ring + uint64_t(slot) * sm_context::kSlotWords, table.data(), table.size() * 8);
     return slot;
+}
+
+// Whether a step that reported an error queued its launch is not known (the error can be an older
+// one of the thread, or that of a timing event behind the launch), so its slots stay pending until
+// the stream has passed it: a launch that still reads a slot that was handed out again would take
+// another layer's addresses, and its late report would set the slot's words back. Holds ring_mu.
+void hold_ring_slot(sm_context* ctx, uint32_t slot, hipStream_t stream) {
+    hipEvent_t& e = ctx->ring_ev[slot];
+    const bool made = e != nullptr || hipEventCreateWithFlags(&e, hipEventDisableTiming) == hipSuccess;
+    ctx->ring_wait[slot].by_event = made && hipEventRecord(e, stream) == hipSuccess;
+    // Without an event the stream is drained here; if that fails too, the slot is never free.
+    if (!ctx->ring_wait[slot].by_event) ctx->ring_pending[slot] = hipStreamSynchronize(stream) != hipSuccess;
 }
 
 void release_ring_slots(sm_segment* seg) {
@@ -957,6 +973,8 @@ void sm_context_destroy(sm_context* ctx) {
     // Teardown is best effort: a failed wait or release leaves nothing the caller can act on.
     for (uint32_t i = 0; i < sm_context::kRingSlots; ++i)
         if (ctx->ring_pending[i]) (void)wait_ring(ctx, i);
+    for (hipEvent_t e : ctx->ring_ev)
+        if (e != nullptr) (void)hipEventDestroy(e);
     if (ctx->ring) (void)hipHostFree(ctx->ring);
     if (ctx->ring_done) (void)hipHostFree(ctx->ring_done);
     if (ctx->side) {
@@ -1049,16 +1067,18 @@ sm_status run_segment(sm_segment* seg, hipStream_t stream, hipEvent_t* ev) {
         }
         side_open = side_open || hs != stream;
         if (st == SM_OK && ev && hipEventRecord(ev[2 * i], hs) != hipSuccess) st = SM_E_DEVICE;
-        if (st == SM_OK && step.run(hs) != hipSuccess) st = SM_E_DEVICE;
+        const bool ran = st == SM_OK;
+        if (ran && step.run(hs) != hipSuccess) st = SM_E_DEVICE;
         if (st == SM_OK && ev && hipEventRecord(ev[2 * i + 1], hs) != hipSuccess) st = SM_E_DEVICE;
         const int s1 = step.ring_slot >= 0 ? step.ring_slot : step.ring_slot2;
         const int s2 = step.ring_slot >= 0 ? step.ring_slot2 : -1;
-        if (s1 >= 0 && st == SM_OK) {  // queued: the slots are free once the launch has reported
+        if (s1 >= 0 && ran) {  // the slots are free once the launch has reported
             std::lock_guard<std::mutex> lk(ctx->ring_mu);
             for (const int slot : {s1, s2}) {
                 if (slot < 0) continue;
-                ctx->ring_wait[slot] = {uint32_t(s1), step.ring_value, step.ring_words};
+                ctx->ring_wait[slot] = {uint32_t(s1), step.ring_value, step.ring_words, false};
                 ctx->ring_pending[slot] = true;
+                if (st != SM_OK) hold_ring_slot(ctx, uint32_t(slot), hs);
             }
         }
     }

@@ -181,3 +181,48 @@ def test_full_ring_waits_for_its_own_launches_only(moe, layer):
     for w, o in zip(ws, want):
         assert w.read_status() == 0
         assert np.array_equal(_out(w).view(np.uint32), o.view(np.uint32))
+
+
+def test_failed_commit_keeps_its_slots(moe, layer):
+    """A commit that reports an error left by an earlier call of the thread has queued its first
+    launch all the same: its slot is not handed out again before that launch has read it (the 64
+    claims behind the failed commit fill every slot with another layer's table)."""
+    import torch
+    print("case slots of a failed commit", flush=True)
+    ctx = moe.Context(0)
+    ws = [layer.DecodeWorkspace(ctx, c, layer.make_inputs(c)) for c in (_decode(layer, moe, 0xC0C3A),
+                                                                       _decode(layer, moe, 0xC0C3B))]
+    main = torch.cuda.current_stream().cuda_stream
+    for w in ws:
+        w.run(main)
+    torch.cuda.synchronize()
+    table = gu.host(ws[0].snap_gu, np.uint8).copy()
+    want = _out(ws[0])
+    ws[0].snap_gu.tensor.fill_(0)
+    rate = _spin_rate()
+    a = torch.cuda.Stream()
+    hip = moe.library()  # resolves the HIP runtime that the library is linked with
+    hip.hipGetLastError()
+    gate = _spin(a, 400, rate)
+    seg = ctx.segment()
+    bufs = ws[0].routed_buffers()
+    ok, err = seg.encode_moe_routed_ffn(ws[0].shape, ws[0].cfg.gate_up_fmt, ws[0].cfg.down_fmt, bufs)
+    assert ok, err
+    assert hip.hipSetDevice(1 << 20) != 0  # an error of the thread, left unread
+    with pytest.raises(RuntimeError, match="SM_E_DEVICE"):
+        seg.commit(a.cuda_stream)
+    assert not gate.query()
+    held = []
+    for _ in range(32):
+        s = ctx.segment()
+        ok, err = ws[1].encode(s)
+        assert ok, err
+        held.append(s)
+    assert gate.query(), "a slot was handed out while the failed commit's launch had not read it"
+    for s in held:
+        s.abort()
+    torch.cuda.synchronize()
+    assert np.array_equal(gu.host(ws[0].snap_gu, np.uint8), table)
+    ws[0].run(main)
+    torch.cuda.synchronize()
+    assert ws[0].read_status() == 0 and np.array_equal(_out(ws[0]).view(np.uint32), want.view(np.uint32))
