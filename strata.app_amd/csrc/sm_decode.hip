@@ -646,10 +646,11 @@ __device__ __forceinline__ void gate_logit_block(const DenseDecode& m) {
 }
 
 // Workgroup bx of nb of one dense mat-vec (a launch of its own, or one part of a fused launch),
-// x_lds its dynamic LDS. NT: the activation rows (1, 2, 4 or 8: the power of two covering them;
-// a row past the last one repeats row 0 and is not stored), so that a chunk's rows are read from
-// LDS together: with a row count known only at run time each of them was a branch and a wait of
-// its own, 80 of them for a router row at T = 8.
+// x_lds its dynamic LDS. NT: the activation rows, so that a chunk's rows are read from LDS
+// together: with a row count known only at run time each of them was a branch and a wait of its
+// own, 80 of them for a router row at T = 8. Every count has its own instance: rounded up to a
+// power of two, the shared down of 5 rows (BF16, 1536 -> 4096) took 11.1 us by events where the
+// run-time count took 9.8 and five rows take 9.1; of 6 rows 11.3, 10.7 and 10.1.
 template <int WT, bool GATE_UP, bool XF32, uint32_t LPR, uint32_t NT>
 __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t bx, uint32_t nb, uint8_t* x_lds) {
     if (GATE_UP && m.gv != nullptr && bx == nb - 1u) {
@@ -697,9 +698,6 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
     for (uint32_t w = 0; w < NW; ++w)
 #pragma unroll
         for (uint32_t t = 0; t < NT; ++t) acc[w][t] = 0.0f;
-    uint32_t xrow[NT];  // first value of each activation row
-#pragma unroll
-    for (uint32_t t = 0; t < NT; ++t) xrow[t] = t < m.rows ? t * m.k : 0u;
     const uint8_t* wr[2] = {m.w0 + uint64_t(row_ok ? row : 0u) * m.k * wbytes,
                             GATE_UP ? m.w1 + uint64_t(row_ok ? row : 0u) * m.k * wbytes : nullptr};
     // Chunks in flight per lane (at most): ten for the router's F32 rows, eight for F16/BF16
@@ -746,7 +744,7 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
                 for (uint32_t t = 0; t < NT; ++t) {
                     float xv[VPC];
                     if (XF32) {
-                        const float* xp = reinterpret_cast<const float*>(x_lds) + xrow[t] + VPC * c;
+                        const float* xp = reinterpret_cast<const float*>(x_lds) + t * m.k + VPC * c;
                         const float4v a = *reinterpret_cast<const float4v*>(xp);
 #pragma unroll
                         for (uint32_t j = 0; j < 4u; ++j) xv[j] = a[j];
@@ -756,7 +754,7 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
                             for (uint32_t j = 0; j < 4u; ++j) xv[(4u + j) % VPC] = b[j];
                         }
                     } else {
-                        const uint8_t* xp = x_lds + (xrow[t] + VPC * c) * 2u;
+                        const uint8_t* xp = x_lds + (t * m.k + VPC * c) * 2u;
                         if (VPC == 8u) {
                             const u32x4 q = *reinterpret_cast<const u32x4*>(xp);
 #pragma unroll
@@ -790,8 +788,7 @@ __device__ __forceinline__ void dense_decode_body(const DenseDecode& m, uint32_t
         const float b = (!GATE_UP && m.bias != nullptr) ? m.bias[row] : 0.0f;
 #pragma unroll
         for (uint32_t t = 0; t < NT; ++t)
-            if (t < m.rows)
-                m.out[uint64_t(t) * m.n_out + row] = GATE_UP ? silu(acc[0][t]) * acc[NW - 1][t] : acc[0][t] + b;
+            m.out[uint64_t(t) * m.n_out + row] = GATE_UP ? silu(acc[0][t]) * acc[NW - 1][t] : acc[0][t] + b;
     }
 }
 
@@ -862,14 +859,20 @@ __host__ __device__ constexpr uint32_t dense_lpr(uint32_t k, uint32_t vpc) {
     return lpr;
 }
 
-// Calls f with the row count's NT and the LPR as constants.
+// Calls f with the row count (1 to 8) and the LPR as constants.
 template <class F>
 hipError_t with_dense_shape(uint32_t rows, uint32_t lpr, F f) {
     auto with_nt = [&](auto lpr_c) {
-        if (rows > 4u) return f(lpr_c, std::integral_constant<uint32_t, 8>());
-        if (rows > 2u) return f(lpr_c, std::integral_constant<uint32_t, 4>());
-        if (rows > 1u) return f(lpr_c, std::integral_constant<uint32_t, 2>());
-        return f(lpr_c, std::integral_constant<uint32_t, 1>());
+        switch (rows) {
+            case 1: return f(lpr_c, std::integral_constant<uint32_t, 1>());
+            case 2: return f(lpr_c, std::integral_constant<uint32_t, 2>());
+            case 3: return f(lpr_c, std::integral_constant<uint32_t, 3>());
+            case 4: return f(lpr_c, std::integral_constant<uint32_t, 4>());
+            case 5: return f(lpr_c, std::integral_constant<uint32_t, 5>());
+            case 6: return f(lpr_c, std::integral_constant<uint32_t, 6>());
+            case 7: return f(lpr_c, std::integral_constant<uint32_t, 7>());
+            default: return f(lpr_c, std::integral_constant<uint32_t, 8>());  // host-checked: at most 8 rows
+        }
     };
     switch (lpr) {
         case 64: return with_nt(std::integral_constant<uint32_t, 64>());

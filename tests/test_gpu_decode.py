@@ -323,7 +323,9 @@ def test_swiglu_combine_bit_exact(moe, orc, gpu_ctx, stream):
 
 # (4, 8, 4096, 4096): the widest rows, whose staged activations need more than 64 KB of LDS
 # (the shared down's F32 hidden rows, 8 x 4096 x 4 bytes).
-@pytest.mark.parametrize("fmt,T,d,Is", [(4, 8, 2560, 640), (5, 3, 4096, 1536), (4, 1, 2048, 512), (4, 8, 4096, 4096)])
+@pytest.mark.parametrize("fmt,T,d,Is", [(4, 8, 2560, 640), (5, 3, 4096, 1536), (4, 1, 2048, 512), (4, 8, 4096, 4096),
+                                         (5, 2, 256, 64), (4, 4, 512, 192), (5, 5, 4096, 1536), (4, 6, 1024, 320),
+                                         (5, 7, 2560, 4096)])
 def test_shared_ffn_against_fp64(moe, orc, gpu_ctx, stream, fmt, T, d, Is):
     print(f"case decode shared fmt={fmt} T={T} d={d} Is={Is}", flush=True)
     gen = moe.synth_normal_bf16 if fmt == moe.BF16 else moe.synth_normal_f16
@@ -387,13 +389,17 @@ def layer_ref(orc, cfg, inp, ws_ids, ws_logits):
 
 
 def _extra_decode(layer, moe, name):
-    """Small layers for the two top-k layouts of the front launch (one token per wave up to 4
-    rows, two per wave above) at expert counts that leave most slots as padding, one without
-    a shared expert."""
+    """Small layers of every row count that the configurations leave out (the front launch's top-k
+    takes tokens w and w + 4 on wave w, and each row count has mat-vec kernels of its own) at
+    expert counts that leave most slots as padding, some without a shared expert."""
     return {"small_t3": layer.LayerConfig("small_t3", 3, 512, 40, 5, 256, 256, moe.Q4_K, moe.Q8_0, moe.F16,
                                           seed=0x5EED0D02),
             "small_t6": layer.LayerConfig("small_t6", 6, 512, 100, 7, 256, 0, moe.Q8_0, moe.Q8_0, moe.F16,
                                           seed=0x5EED0D03),
+            "small_t5": layer.LayerConfig("small_t5", 5, 512, 72, 6, 256, 256, moe.Q4_K, moe.Q8_0, moe.F16,
+                                          seed=0x5EED0D06),
+            "small_t7": layer.LayerConfig("small_t7", 7, 512, 40, 5, 256, 512, moe.Q8_0, moe.Q8_0, moe.BF16,
+                                          seed=0x5EED0D07),
             "small_t2": layer.LayerConfig("small_t2", 2, 512, 64, 8, 256, 256, moe.Q4_K, moe.Q8_0, moe.F16,
                                           seed=0x5EED0D04),
             "small_t1": layer.LayerConfig("small_t1", 1, 512, 40, 5, 256, 0, moe.Q4_K, moe.Q8_0, moe.F16,
@@ -401,7 +407,7 @@ def _extra_decode(layer, moe, name):
 
 
 @pytest.mark.parametrize("name", ["window_t1", "window_t8", "full_layer_t8", "low_bit_t4", "small_t3", "small_t6",
-                                  "small_t2", "small_t1"])
+                                  "small_t2", "small_t1", "small_t5", "small_t7"])
 def test_decode_layer(moe, layer, orc, gpu_ctx, stream, name):
     print(f"case decode layer {name}", flush=True)
     cfg = layer.DECODE_CONFIGS[name] if name in layer.DECODE_CONFIGS else _extra_decode(layer, moe, name)
