@@ -828,12 +828,13 @@ __global__ __launch_bounds__(256) void decode_front_kernel(DecodePlanArgs a, con
         __shared__ uint2 cand[4][kTopkCand];
         const uint32_t wave = threadIdx.x >> 6;
         float v[8], v4[8];
-        topk_load(a.logits, a.rows, a.n_experts, wave, v);
-        if (NT > 4u) topk_load(a.logits, a.rows, a.n_experts, wave + 4u, v4);
-        topk_token(v, a.route_ids, a.route_weights, a.rows, a.n_experts, a.top_k, 0, nullptr, wave, cand[wave], ids_s);
+        topk_load<8, true>(a.logits, a.rows, a.n_experts, wave, v);
+        if (NT > 4u) topk_load<8, true>(a.logits, a.rows, a.n_experts, wave + 4u, v4);
+        topk_token<8, true>(v, a.route_ids, a.route_weights, a.rows, a.n_experts, a.top_k, 0, nullptr, wave, cand[wave],
+                            ids_s);
         if (NT > 4u)
-            topk_token(v4, a.route_ids, a.route_weights, a.rows, a.n_experts, a.top_k, 0, nullptr, wave + 4u, cand[wave],
-                       ids_s);
+            topk_token<8, true>(v4, a.route_ids, a.route_weights, a.rows, a.n_experts, a.top_k, 0, nullptr, wave + 4u,
+                                cand[wave], ids_s);
         __syncthreads();
         moe_plan_body(a, ids_s);
         return;

@@ -1,5 +1,7 @@
 // Router GEMM, softmax top-k, stable expert grouping, F16 row gather, and the plan /
 // destination validators for gfx950.
+#include <type_traits>
+
 #include "sm_device.h"
 #include "sm_launch.h"
 #include "sm_topk.h"
@@ -240,17 +242,32 @@ __global__ __launch_bounds__(kRouterThreads) void router_gemm_kernel(const _Floa
     }
 }
 
-template <int NV>
+template <int NV, bool WAVE>
 __global__ __launch_bounds__(256) void route_topk_kernel(const float* __restrict__ logits,
                                                          int32_t* __restrict__ ids,
                                                          float* __restrict__ weights,
                                                          uint32_t rows, uint32_t E, uint32_t K,
                                                          int divide, uint32_t* __restrict__ hist) {
-    __shared__ uint2 cand[4][kTopkCand];
-    const uint32_t wave = threadIdx.x >> 6, t = blockIdx.x * 4u + wave;
+    __shared__ uint2 cand[4][WAVE ? kTopkCand : 1u];
+    const uint32_t wave = threadIdx.x >> 6;
+    const uint32_t t = WAVE ? blockIdx.x * 4u + wave : blockIdx.x * 8u + (threadIdx.x >> 5);
     float v[NV];
-    topk_load(logits, rows, E, t, v);
-    topk_token(v, ids, weights, rows, E, K, divide, hist, t, cand[wave], nullptr);
+    topk_load<NV, WAVE>(logits, rows, E, t, v);
+    topk_token<NV, WAVE>(v, ids, weights, rows, E, K, divide, hist, t, cand[wave], nullptr);
+}
+
+// Whether the top-k of many tokens takes two per wave in rounds instead of one per wave with
+// counted ranks. Two per wave halve the instructions of everything but the rounds, and the rounds
+// cost K times the slots; up to 1024 tokens (one wave per SIMD) only a token's own chain counts.
+// Launch times (events, us), two per wave against one: 4096 tokens, 128 experts, K = 10 7.1 and
+// 8.0, 256, 8 7.6 and 8.3, 512, 4 7.7 and 8.9, 512, 10 10.3 and 9.9, 512, 16 12.8 and 11.2; 16384
+// tokens, 128, 4 9.1 and 13.6, 512, 10 23.9 and 23.0; 2048 tokens, 256, 6 6.4 and 6.5, 256, 10 7.4
+// and 7.0, 512, 6 7.9 and 7.2; where K is past the count, 4096 tokens, 128, 32 12.2 and 21.5.
+inline bool topk_by_half_wave(uint32_t rows, uint32_t E, uint32_t K) {
+    if (rows <= 1024u) return false;
+    if (K > kTopkCountK && E > kTopkCand) return true;
+    const uint32_t work = K * ((E + 63u) / 64u);
+    return rows <= 3072u ? K < 16u && (K < 6u || work <= 24u) : work <= 64u;
 }
 
 // ---------------------------------------------------------------------------------------
@@ -915,11 +932,24 @@ hipError_t launch_router_gemm(const _Float16* x, const float* w, const float* bi
 hipError_t launch_route_topk(const float* logits, int32_t* ids, float* weights, uint32_t rows,
                              uint32_t E, uint32_t K, int divide, hipStream_t s, uint32_t* hist) {
     if (E == 0u || E > 512u || K == 0u || K > 32u || K > E) return hipErrorInvalidValue;
-    const uint32_t blocks = (rows + 3u) / 4u, nv = (E + 63u) / 64u;
-    if (nv <= 1) route_topk_kernel<1><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-    else if (nv <= 2) route_topk_kernel<2><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-    else if (nv <= 4) route_topk_kernel<4><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
-    else route_topk_kernel<8><<<blocks, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
+    auto go = [&](auto nv, auto wave) {
+        const uint32_t per = wave.value ? 4u : 8u;  // tokens per workgroup
+        route_topk_kernel<nv.value, wave.value><<<(rows + per - 1u) / per, 256, 0, s>>>(logits, ids, weights, rows, E, K, divide, hist);
+    };
+    if (topk_by_half_wave(rows, E, K)) {
+        const uint32_t nv = (E + 31u) / 32u;
+        if (nv <= 1) go(std::integral_constant<int, 1>(), std::false_type());
+        else if (nv <= 2) go(std::integral_constant<int, 2>(), std::false_type());
+        else if (nv <= 4) go(std::integral_constant<int, 4>(), std::false_type());
+        else if (nv <= 8) go(std::integral_constant<int, 8>(), std::false_type());
+        else go(std::integral_constant<int, 16>(), std::false_type());
+    } else {
+        const uint32_t nv = (E + 63u) / 64u;
+        if (nv <= 1) go(std::integral_constant<int, 1>(), std::true_type());
+        else if (nv <= 2) go(std::integral_constant<int, 2>(), std::true_type());
+        else if (nv <= 4) go(std::integral_constant<int, 4>(), std::true_type());
+        else go(std::integral_constant<int, 8>(), std::true_type());
+    }
     return hipGetLastError();
 }
 

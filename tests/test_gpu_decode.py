@@ -454,6 +454,49 @@ def test_decode_layer(moe, layer, orc, gpu_ctx, stream, name):
     assert np.array_equal(gu.host(ws.out, np.float32).reshape(T, d).view(np.uint32), first.view(np.uint32))
 
 
+@pytest.mark.parametrize("T,E,K", [(4, 512, 10), (5, 512, 10), (8, 512, 10), (8, 128, 10), (2, 512, 32), (3, 100, 24)])
+def test_decode_layer_route_edges(moe, layer, orc, gpu_ctx, stream, T, E, K):
+    """The front launch's top-k and plan on crafted logits: one-hot tokens pick router columns, so
+    token t's logits are its row exactly. Equal values around the 64 candidates that are ranked by
+    counting, so that a token that takes the rounds follows or precedes a counted one on the same
+    wave (tokens w and w + 4); then one bias row for all tokens: all equal, with NaN and with
+    infinities (the plan's ids must stay distinct and in range)."""
+    print(f"case decode route edges T={T} E={E} K={K}", flush=True)
+    import torch
+    cfg = layer.LayerConfig("dec_edges", T, 256, E, K, 64, 0, moe.Q8_0, moe.Q8_0, moe.F16, seed=0x5EED0D08)
+    inp = layer.make_inputs(cfg)
+    rng = np.random.default_rng(T * 1000 + E)
+    counts = [n for n in (65, K, 64, E, 63, E, K + 1, 65) if n <= E]
+    rows = np.full((T, E), -1.0, np.float32) - rng.random((T, E)).astype(np.float32)
+    for t in range(T):
+        rows[t, rng.permutation(E)[:counts[t % len(counts)]]] = 2.0
+    zero = np.zeros((E, cfg.hidden), np.float32)
+    onehot = zero.copy()
+    onehot[:, :T] = rows.T
+    x = np.zeros((inp.x.shape[0], cfg.hidden), np.float16)
+    x[np.arange(T), np.arange(T)] = 1.0
+    inp.x = x.view(inp.x.dtype)
+    nan = rng.standard_normal(E).astype(np.float32)
+    nan[::3] = np.nan
+    low = np.full(E, -np.inf, np.float32)
+    low[5] = 1.0
+    for what, router, bias in (("counts", onehot, None), ("equal", zero, np.zeros(E, np.float32)), ("nan", zero, nan),
+                               ("one finite", zero, low), ("infinite", zero, -low)):
+        inp.w_router, inp.bias = router, bias
+        ws = layer.DecodeWorkspace(gpu_ctx, cfg, inp)
+        ws.run(stream)
+        torch.cuda.synchronize()
+        logits = gu.host(ws.logits, np.float32).reshape(T, E)
+        if what == "counts":
+            assert np.array_equal(logits, rows)
+        ids, w = orc.route(logits, K, False)
+        assert np.array_equal(gu.host(ws.ids, np.int32).reshape(T, K), ids), what
+        assert np.array_equal(gu.host(ws.route_w, np.float32).reshape(T, K).view(np.uint32), w.view(np.uint32)), what
+        plan, rc = orc.moe_plan(ids, E)
+        assert rc == 0 and np.array_equal(gu.host(ws.plans, np.uint8), plan), what
+        assert ws.read_status() == 0
+
+
 @pytest.mark.parametrize("name", ["window_t1", "window_t8"])
 def test_decode_layer_null_expert_address(moe, layer, orc, gpu_ctx, stream, name):
     """A routed expert without an up matrix: status bit 0, its group's gate/up rows, SwiGLU rows

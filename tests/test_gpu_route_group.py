@@ -25,11 +25,14 @@ def _route_case(moe, orc, ctx, stream, logits, K, divide):
     return gu.host(ids, np.int32).reshape(T, K), gu.host(w, np.float32).reshape(T, K)
 
 
-# Up to 1024 tokens the kernel takes one token per wave, above that two per wave: both layouts
-# meet every slot count (E up to 64 / 128 / 256 / 512 per wave, 32 / 64 / 128 / 256 / 512 per
-# half-wave) and the reference's golden rows (K = 10, E = 512 in each layout).
+# Two layouts, one token per wave (ranks counted among the candidates, or rounds past K = 20) and
+# two tokens per wave (rounds); many tokens take the second where K times the slots is small, or
+# K is past 20. Both meet every slot count (E up to 64 / 128 / 256 / 512 per wave, 32 / 64 / 128 /
+# 256 / 512 per half-wave) and the reference's golden rows.
 @pytest.mark.parametrize("T,E,K", [(64, 16, 4), (4096, 512, 10), (1000, 256, 8), (37, 40, 5), (9, 512, 32),
-                                   (8, 512, 10), (300, 100, 6), (1025, 100, 6), (2000, 40, 10), (1500, 200, 10)])
+                                   (8, 512, 10), (300, 100, 6), (1025, 100, 6), (2000, 40, 10), (1500, 200, 10),
+                                   (1025, 16, 4), (4096, 256, 10), (5000, 512, 8), (1100, 512, 21), (3072, 64, 16),
+                                   (3073, 64, 16)])
 @pytest.mark.parametrize("divide", [True, False])
 def test_route_topk_bit_exact(moe, orc, gpu_ctx, stream, T, E, K, divide):
     print(f"case route T={T} E={E} K={K} divide={divide}", flush=True)
@@ -52,6 +55,41 @@ def test_route_topk_bit_exact(moe, orc, gpu_ctx, stream, T, E, K, divide):
         gold = rp.NONUNIFORM_DIVIDE_BITS if divide else rp.NONUNIFORM_MULTIPLY_BITS
         assert list(w[2].view(np.uint32)) == gold
         assert list(w[0].view(np.uint32)) == rp.EQUAL_WEIGHT_BITS
+
+
+def _edge_rows(rng, E, K):
+    """Rows that put a chosen number of equal values at the top (63, 64 and 65 around the 64
+    candidates that are ranked by counting, all of them equal, and ties on both sides of rank K),
+    and rows where K - 1 larger values leave one rank to equal ones of the same and of other lanes."""
+    rows = []
+    for n in sorted({K, K + 1, 63, 64, 65, E - 1, E}):
+        if n <= E:
+            row = rng.permutation(E).astype(np.float32) * np.float32(-0.01) - np.float32(1.0)
+            row[rng.permutation(E)[:n]] = 2.0
+            rows.append(row)
+    for step in (1, 31, 32, 33):
+        row = rng.permutation(E).astype(np.float32) * np.float32(-0.01) - np.float32(1.0)
+        tied = (int(rng.integers(E)) + step * np.arange(3)) % E
+        top = [e for e in rng.permutation(E) if e not in tied][:K - 1]
+        row[top] = 3.0 + np.arange(len(top), dtype=np.float32) * np.float32(0.125)
+        row[tied] = 2.0
+        rows.append(row)
+    return np.stack(rows)
+
+
+# 1100 rows: two tokens per wave for K = 1 and 4 at every E, 10 at up to 128 experts, 21 and 32 at
+# more than 64; one per wave otherwise.
+@pytest.mark.parametrize("T", [11, 1100])
+@pytest.mark.parametrize("E,K", [(65, 1), (65, 10), (65, 32), (128, 10), (128, 20), (128, 21), (512, 4), (512, 10),
+                                 (512, 20), (512, 21), (512, 32), (33, 32), (64, 32)])
+def test_route_topk_ties_and_candidate_count(moe, orc, gpu_ctx, stream, T, E, K):
+    print(f"case route ties T={T} E={E} K={K}", flush=True)
+    rows = _edge_rows(np.random.default_rng(E * 64 + K), E, K)
+    logits = rows[np.arange(T) % len(rows)]
+    ids, w = _route_case(moe, orc, gpu_ctx, stream, logits, K, True)
+    ids_ref, w_ref = orc.route(logits, K, True)
+    assert np.array_equal(ids, ids_ref)
+    assert np.array_equal(w.view(np.uint32), w_ref.view(np.uint32))
 
 
 @pytest.mark.parametrize("E", [256, 512])
