@@ -483,8 +483,19 @@ inline TilePlan tile_plan(uint32_t k, uint32_t n_out) {
 // 16.2 us as 256, and 128 row tiles of 8 (d = 2048, Q8_0) 65 -> 49 us. Past one item per
 // workgroup a split only re-reads activations: halving on to two items each measured 110.5 ->
 // 116 us (440 row tiles) and 49 -> 51 us (128), to four 175 -> 187 us (515).
-__device__ __forceinline__ uint32_t split_npi(uint32_t tiles, uint32_t n_ntiles, uint32_t npi) {
-    while (npi > 1u && tiles * ((n_ntiles + npi - 1u) / npi) < gridDim.x) npi = (npi + 1u) >> 1;
+// `after`: wide items that the same workgroups draw once their tiles are done (a down stage). There
+// the split goes on only while every item still has a workgroup of its own: past that the tile
+// items and the wide items, which ran side by side, run one after the other (92 wide items and 59
+// row tiles of 4 column tiles, d = 1024, K = 512: 33.1 us as 59 items, 49.8 as 236; 72 and 131 of
+// 8, Q8_0: 64.5 as 131, 81.0 as 262). A gate/up stage draws its tiles behind the wide items, and
+// shorter ones fill its end better (216 wide items and 51 row tiles: 81.6 us as 102 items, 63.0 as
+// 204).
+__device__ __forceinline__ uint32_t split_npi(uint32_t tiles, uint32_t n_ntiles, uint32_t npi, uint32_t after) {
+    while (npi > 1u) {
+        const uint32_t half = (npi + 1u) >> 1, items = tiles * ((n_ntiles + npi - 1u) / npi);
+        if (after == 0u ? items >= gridDim.x : tiles * ((n_ntiles + half - 1u) / half) + after > gridDim.x) break;
+        npi = half;
+    }
     return npi;
 }
 
@@ -526,7 +537,8 @@ __device__ void zero_tile_slots(const RoutedGemm& g, uint32_t n_ntiles, uint32_t
 // HALF (direct form): K ends with a half slab, resident as well.
 template <class Frag, int MODE, int NF, bool RESIDENT, bool DYNAMIC, bool HALF = false>
 __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, NF, HALF>& sm, const uint32_t* s_pref,
-                                           uint32_t n_ntiles, uint32_t npi_launch, const int32_t* s_grp) {
+                                           uint32_t n_ntiles, uint32_t npi_launch, const int32_t* s_grp,
+                                           uint32_t after = 0u) {
     constexpr bool dynamic = DYNAMIC;
     using S = Staged<MODE, NF>;
     using WC = WeightCopy<Frag, MODE, NF>;
@@ -535,7 +547,7 @@ __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, N
     auto& sa = sm.sa;
     auto& sw = sm.sw;
     uint32_t* s_dst = sm.s_dst;
-    const uint32_t npi = split_npi(s_pref[512], n_ntiles, npi_launch), n_chunks = (n_ntiles + npi - 1u) / npi;
+    const uint32_t npi = split_npi(s_pref[512], n_ntiles, npi_launch, after), n_chunks = (n_ntiles + npi - 1u) / npi;
     const uint32_t items = s_pref[512] * n_chunks;
     const uint32_t per = (items + 7u) >> 3, x = blockIdx.x & 7u, P = gridDim.x >> 3;
     const uint32_t i_end = (x + 1u) * per < items ? (x + 1u) * per : items;

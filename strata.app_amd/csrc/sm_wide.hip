@@ -596,7 +596,7 @@ __global__ __launch_bounds__(kWideThreads) void routed_stage_kernel(RoutedGemm g
             tile_items<Frag, MODE, 2, RESIDENT, false, HALF>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
         }
     } else {
-        tile_items<Frag, MODE, 2, RESIDENT, false, HALF>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp);
+        tile_items<Frag, MODE, 2, RESIDENT, false, HALF>(g, sm.t, s_pref_t, n_ntiles, npi, s_grp, U * n_ct);
         if (U > 0u) {
             __syncthreads();  // the tile phase's LDS is free
             // Workgroups leave the tile phase at different times: the wide items are drawn.

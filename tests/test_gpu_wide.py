@@ -45,6 +45,21 @@ def test_wide_only_partial_units(moe, layer, orc, gpu_ctx, stream):
     assert counts.min() >= 128
 
 
+# Few row tiles beside wide units: the down tiles split by column tile while each item and each wide
+# item has a workgroup (here to 2 and to 1 of 4 column tiles, and, streamed, 2 of 4 to 1), the
+# gate/up tiles until every workgroup has one.
+@pytest.mark.parametrize("rows,zipf,ff,down", [(400, 0.6, 512, "Q4_K"), (300, 1.1, 256, "Q8_0"), (300, 0.6, 1024, "Q2_K")])
+def test_split_tiles_beside_wide_units(moe, layer, orc, gpu_ctx, stream, rows, zipf, ff, down):
+    print(f"case wide beside split tiles rows {rows} zipf {zipf} I {ff} down {down}", flush=True)
+    cfg = layer.LayerConfig("wide_split", rows, 1024, 64, 8, ff, 0, moe.Q4_K, getattr(moe, down), moe.F16, zipf_s=zipf,
+                            seed=205)
+    ws = _check_layer(moe, layer, orc, gpu_ctx, stream, cfg)
+    counts = np.bincount(gu.host(ws.ids, np.int32), minlength=cfg.n_experts)
+    wide = int((-(-counts[counts >= 128] // 256)).sum()) * 4
+    tiles = int((-(-counts[counts < 128] // 64)).sum())
+    assert wide > 0 and 0 < 2 * tiles + wide <= 256
+
+
 def _victim_rows(orc, ws, cfg, victim):
     ids = gu.host(ws.ids, np.int32)
     g = orc.grouping(ids.reshape(cfg.rows, cfg.top_k), cfg.n_experts)
