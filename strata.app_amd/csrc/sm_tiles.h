@@ -438,10 +438,17 @@ struct StagedBuffers {
 // LDS of the staged tile kernels: the activation slabs (or the resident tile, with HALF its
 // half slab), the weight image(s), the tile's destination rows (down) and the next dynamically
 // drawn item.
-template <class Frag, int NF, bool HALF = false>
-struct TileSmem {
+template <bool HALF>
+struct SlabSmem {
     _Float16 sa[2][64 * kSlab] __attribute__((aligned(1024)));
-    _Float16 sh[HALF ? 64 * kSlab / 2 : 8] __attribute__((aligned(1024)));
+};
+template <>
+struct SlabSmem<true> {
+    _Float16 sa[2][64 * kSlab] __attribute__((aligned(1024)));
+    _Float16 sh[64 * kSlab / 2] __attribute__((aligned(1024)));
+};
+template <class Frag, int NF, bool HALF = false>
+struct TileSmem : SlabSmem<HALF> {
     uint8_t sw[StagedBuffers<Frag, NF>::kWBuf][StagedBuffers<Frag, NF>::kImage] __attribute__((aligned(1024)));
     uint32_t s_dst[64];  // down: destination row of each tile row
     uint32_t s_next;
@@ -608,7 +615,7 @@ __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, N
         for (uint32_t sb = 0; sb < n_slabs; ++sb) issue_slab(asrc, sb * kSlab, sa[sb], wave);
     constexpr bool DIRECT = DirectWeights<Frag, MODE, RESIDENT>::value;
     static_assert(!HALF || DIRECT, "the half slab belongs to the direct form");
-    if (HALF) issue_half_slab(g, t, n_slabs * kSlab, sm.sh, wave, lane);
+    if constexpr (HALF) issue_half_slab(g, t, n_slabs * kSlab, sm.sh, wave, lane);
     if constexpr (DIRECT) {
         // Steps are (column tile, half f): the wave's 16 weight rows of fragment f, rows
         // 128 f + 16 wave + n of the column tile, with every slab of them loaded at once, so a
