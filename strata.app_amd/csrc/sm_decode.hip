@@ -425,7 +425,6 @@ __global__ __launch_bounds__(256, 4) void moe_matvec_kernel(DecodeMatvec m) {  /
     extern __shared__ uint32_t act_s[];
     const uint32_t tid = threadIdx.x, lane = tid & 63u, wave = tid >> 6;
     const uint32_t g = blockIdx.y;
-    const DecodePlan* P = reinterpret_cast<const DecodePlan*>(m.plan);
     if (g >= 80u) return;
     // A plan whose header is unusable: workgroup (0, 0) reports it and zeroes every output row
     // this stage could have written.

@@ -34,8 +34,13 @@ namespace {
 // room. The sums keep their order, so the logits are the same bits. Routing alone: 100 tokens
 // 26.4 -> 25.4 us (512 experts, d 2048), 500 tokens 38.9 -> 36.8 (256, 4096), 800 tokens 32.8 ->
 // 31.7; layers: 513 tokens of 128 experts 190.5 -> 186.9, 500 of 512 experts 358.9 -> 353.2, 800
-// 378.6 -> 377.3 and without a shared expert the same. At 2000 tokens of 128 experts the ring
-// shuts the shared expert's workgroups out of more CUs and the layer went 394 -> 399.5 us.
+// 378.6 -> 377.3 and without a shared expert the same. What ends it is LDS: one workgroup of 120 KB
+// per CU where two of the plain form fit, so routing alone gains while there are at most 256
+// workgroups (128 experts, 2000 tokens: 252 of them, 42.5 -> 41.3; 512, 1000: 35.5 -> 34.1) and loses
+// past that (512, 1500: 45.6 -> 49.0), and beside a shared expert, whose workgroups want the same
+// CUs, it loses earlier: layers with one of 512 columns, 1000 tokens of 128 experts 272.9 -> 268.5,
+// 1400 357.2 -> 365.5, of 256 experts 413.2 -> 422.9, 2000 of 64 to 256 experts 1 to 1.5% more. 800
+// lies below every loss measured.
 // ---------------------------------------------------------------------------------------
 constexpr int kRouterCols = 64;
 constexpr int kRouterThreads = 512;
@@ -912,6 +917,7 @@ __global__ __launch_bounds__(256) void destination_validate_kernel(const int32_t
 
 hipError_t launch_router_gemm(const _Float16* x, const float* w, const float* bias, float* logits,
                               uint32_t rows, uint32_t d, uint32_t E, hipStream_t s, const RouterPrep* prep) {
+    if (d % 256u != 0u) return hipErrorInvalidValue;  // whole stages and stage pairs (host-checked)
     const RouterPrep rp = prep != nullptr ? *prep : RouterPrep{};
     // The largest token tile that still launches at least one workgroup per CU (256), so
     // each expert's weights are split as few times as the layer allows.
@@ -921,7 +927,7 @@ hipError_t launch_router_gemm(const _Float16* x, const float* w, const float* bi
         router_gemm_kernel<128, 1><<<dim3((rows + 127) / 128, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
     } else if (blocks(64) >= 256u) {
         router_gemm_kernel<64, 1><<<dim3((rows + 63) / 64, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
-    } else if (rows <= kRouterPairRows && d % 128u == 0u) {
+    } else if (rows <= kRouterPairRows) {  // d % 128 == 0 as well
         router_gemm_kernel<32, 2><<<dim3((rows + 31) / 32, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);
     } else {
         router_gemm_kernel<32, 1><<<dim3((rows + 31) / 32, ecols), kRouterThreads, 0, s>>>(x, w, bias, logits, rows, d, E, rp);

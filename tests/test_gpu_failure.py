@@ -14,8 +14,12 @@ import ref_patterns as rp
 pytestmark = pytest.mark.gpu
 
 
-def _small_layer(moe, layer, ctx):
-    cfg = layer.LayerConfig("fail", 32, 256, 16, 4, 128, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=91)
+# 32 rows group in one workgroup; 5200 rows are 82 histogram tiles, past the 80 that do.
+BOTH_GROUPINGS = pytest.mark.parametrize("rows", [32, 5200])
+
+
+def _small_layer(moe, layer, ctx, rows=32):
+    cfg = layer.LayerConfig("fail", rows, 256, 16, 4, 128, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=91)
     inp = layer.make_inputs(cfg)
     return cfg, inp, layer.LayerWorkspace(ctx, cfg, inp)
 
@@ -112,11 +116,12 @@ def test_swiglu_and_combine_bit_exact(moe, orc, gpu_ctx, stream):
     assert np.array_equal(gu.host(bo, np.float32).reshape(T, d).view(np.uint32), ref0.view(np.uint32))
 
 
-def test_full_layer_clears_both_status_words_and_reports_null_address(moe, layer, orc, gpu_ctx, stream):
+@BOTH_GROUPINGS
+def test_full_layer_clears_both_status_words_and_reports_null_address(moe, layer, orc, gpu_ctx, stream, rows):
     """The full layer checks its plan once for both expert stages: both status words start
     cleared, and a missing weight address is still reported by the gate/up tiles."""
     print("case failure full layer status words", flush=True)
-    cfg, inp, ws = _small_layer(moe, layer, gpu_ctx)
+    cfg, inp, ws = _small_layer(moe, layer, gpu_ctx, rows)
     ws.status.tensor.fill_(-1)                       # stale bits from an earlier failure
     ws.run_layer(stream)
     assert ws.read_status(stream) == (0, 0, 0)
@@ -144,14 +149,15 @@ def _foreign(gpu_ctx, tensor, dtype, edit):
     return gpu_ctx.register(gu.dev(host))
 
 
+@BOTH_GROUPINGS
 @pytest.mark.parametrize("fault", ["repeat", "out_of_range"])
-def test_full_layer_checks_destinations_in_the_gather(moe, layer, orc, gpu_ctx, stream, fault):
+def test_full_layer_checks_destinations_in_the_gather(moe, layer, orc, gpu_ctx, stream, fault, rows):
     """A full layer whose down stage reads a destination map other than the grouping's: the
     gather launch marks it in the bitset, a repeated or out-of-range entry sets bit 1 of the
     down status only, and the down tiles write zeros (metal_prefill_moe_full_pipeline_test.mm:
     1081-1104 permutation faults)."""
     print(f"case failure full layer destination {fault}", flush=True)
-    cfg, inp, ws = _small_layer(moe, layer, gpu_ctx)
+    cfg, inp, ws = _small_layer(moe, layer, gpu_ctx, rows)
     ws.run_layer(stream)
     N = cfg.rows * cfg.top_k
 
@@ -179,12 +185,13 @@ def test_full_layer_checks_destinations_in_the_gather(moe, layer, orc, gpu_ctx, 
     assert ws.read_status(stream) == (0, 0, 0)
 
 
-def test_full_layer_checks_a_foreign_plan_in_the_gather(moe, layer, orc, gpu_ctx, stream):
+@BOTH_GROUPINGS
+def test_full_layer_checks_a_foreign_plan_in_the_gather(moe, layer, orc, gpu_ctx, stream, rows):
     """Both expert stages bound to one plan and tile list other than the grouping's, with a
     broken tile chain: the plan check in the gather launch sets bit 1 of both status words and
     both stages write zeros (prefill_moe.metal:603-733)."""
     print("case failure full layer foreign plan", flush=True)
-    cfg, inp, ws = _small_layer(moe, layer, gpu_ctx)
+    cfg, inp, ws = _small_layer(moe, layer, gpu_ctx, rows)
     ws.run_layer(stream)
     plan2 = _foreign(gpu_ctx, ws.plan, np.uint8, lambda p: None)
 

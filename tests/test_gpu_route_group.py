@@ -108,6 +108,41 @@ def test_grouping_one_workgroup_limits(moe, orc, gpu_ctx, stream, pattern, T, E)
     _check_grouping_gather(moe, orc, gpu_ctx, stream, pattern, T, E)
 
 
+# With a residency table (experts at or above 0 are resident): the plan's per-group flags, its miss
+# count and skip flag, on both sides of 80 tiles.
+@pytest.mark.parametrize("T,E", [(26, 64), (410, 512), (2048, 512), (2049, 512), (2049, 40), (4096, 300)])
+@pytest.mark.parametrize("cold", ["some", "none", "unused"])
+def test_grouping_residency(moe, orc, gpu_ctx, stream, T, E, cold):
+    print(f"case grouping residency T={T} E={E} cold={cold}", flush=True)
+    K, d = 10, 256
+    rng = np.random.default_rng(T + E)
+    ids = np.stack([rng.permutation(E - 1)[:K] for _ in range(T)]).astype(np.int32)  # the last expert is never used
+    resident = rng.integers(0, 1000, (2, E)).astype(np.int32)
+    resident[1, E - 1] = -1 if cold != "none" else 0
+    if cold == "some":
+        resident[1, ::3] = -1
+    resident[0] = -1  # the other layer's table must not be read
+    reg, N, shape = gpu_ctx.register, T * K, moe.Shape(T, d, E, K, 64, 0)
+    b_ids, b_x, b_res = reg(gu.dev(ids)), reg(gu.dev(np.zeros((T, d), np.uint16))), reg(gu.dev(resident))
+    hist, plan = reg(gu.poison(moe.histogram_bytes(shape))), reg(gu.poison(moe.PLAN_SLOT_BYTES))
+    tiles, xs = reg(gu.poison(moe.tiles_bytes(shape))), reg(gu.poison(N * d * 2))
+    src, dst = reg(gu.poison(N * 4)), reg(gu.poison(N * 4))
+    b = moe.GroupingBuffers(b_ids.view(), b_x.view(), hist.view(), plan.view(), tiles.view(), src.view(), dst.view(),
+                            xs.view(), b_res.view(), 1)
+    gu.run(gpu_ctx, stream, lambda s: s.encode_prefill_moe_grouping(shape, b))
+    ref = orc.grouping(ids, E)
+    want = ref["plan"].copy()
+    w = want[:6180].view(np.int32)
+    groups = int(w[0])
+    flags = (resident[1][w[8:8 + groups]] >= 0).astype(np.int32)
+    w[520:520 + groups] = flags
+    w[2] = groups - int(flags.sum())
+    w[3] = int(w[2] == 0)
+    assert (w[2] > 0) == (cold == "some")
+    assert np.array_equal(gu.host(plan, np.uint8), want)
+    assert np.array_equal(gu.host(dst, np.int32), ref["dst"]) and np.array_equal(gu.host(src, np.int32), ref["src"])
+
+
 # The scan keeps up to 16 of its 256-entry tiles per thread in registers (512 tiles: N = 131072
 # entries); longer columns take its re-reading loop. 13107 tokens x 10 is 512 tiles, 16384 x 10
 # is 640.

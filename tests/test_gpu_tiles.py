@@ -32,12 +32,12 @@ def _cases(layer, moe):
         "q80_2slab": C("tiles_q80b", 128, 256, 8, 2, 512, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=303),
         # gate/up Q4_K: 3 column tiles; down K = 384: one whole slab and a half one
         "odd_tiles": C("tiles_odd", 192, 512, 12, 2, 384, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=304),
-        # 512 gate/up items (128 groups x 4 column tiles) on at most 256 workgroups: each
-        # workgroup runs items back to back, the next one's copies issued by the current one
         # 128 row tiles x 5 down column tiles on 256 workgroups: items of 3 and 2 column tiles
         "split_items": C("tiles_split", 256, 1280, 128, 8, 512, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=306),
         # the same on the streamed path: 2 column tiles per item at the launch, split to 1
         "split_stream": C("tiles_split_s", 128, 1024, 32, 4, 1024, 0, moe.Q2_K, moe.Q4_K, moe.F16, seed=307),
+        # 512 gate/up items (128 groups x 4 column tiles) on at most 256 workgroups: each
+        # workgroup runs items back to back, the next one's copies issued by the current one
         "many_items": C("tiles_many", 1024, 1280, 128, 8, 512, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=305),
     }
 
@@ -125,8 +125,9 @@ def test_tile_broken_destination_zeroes_parts(moe, layer, orc, gpu_ctx, stream):
 
 @pytest.mark.parametrize("ff", [64, 128, 192, 320])
 def test_short_reduction_rows(moe, layer, orc, gpu_ctx, stream, ff):
-    """Down reductions that end inside a 256-value slab: the lanes past K stay inside their row
-    (rows of 64 to 192 values are shorter than the slab that the other lanes cover)."""
+    """Down reductions that end inside a 256-value slab (rows of 64 to 192 values are shorter than
+    the slab that the other lanes cover): the lanes past K must contribute nothing. What they
+    read, the start of their row, shows in no output."""
     print(f"case tiles short reduction {ff}", flush=True)
     cfg = layer.LayerConfig("tiles_short", 96, 256, 12, 2, ff, 0, moe.Q8_0, moe.Q8_0, moe.F16, seed=311)
     _check_layer(moe, layer, orc, gpu_ctx, stream, cfg)
