@@ -484,12 +484,14 @@ inline TilePlan tile_plan(uint32_t k, uint32_t n_out) {
     return p;
 }
 
-// Column tiles per item for `tiles` row tiles on this grid: the launch's npi, halved while there
-// would be fewer items than workgroups. What few row tiles cost is then the longest item, not
-// bandwidth: 64 row tiles of 4 column tiles (d = 1024, I = 512) took 31.4 us as 64 down items and
-// 16.2 us as 256, and 128 row tiles of 8 (d = 2048, Q8_0) 65 -> 49 us. Past one item per
-// workgroup a split only re-reads activations: halving on to two items each measured 110.5 ->
-// 116 us (440 row tiles) and 49 -> 51 us (128), to four 175 -> 187 us (515).
+// Column tiles per item for `tiles` row tiles on this grid (n_chunks: items per row tile): the
+// launch's npi, halved while that shortens the stage. What few row tiles cost is the longest
+// workgroup's items, not bandwidth: rounds of items times an item's column tiles plus about two
+// more for its start (64 row tiles of 4, d = 1024, K = 512: 25.3 us as 64 down items, 13.2 as 256;
+// 128 of 8, d = 2048, Q8_0: 48.8 as 128, 34.0 as 256). A split into a second round of items loses
+// (140 of 4, Q8_0: 27.1 -> 31.2; 180 of 8: 60.1 -> 62.8), a third round of half the length for two
+// whole ones gains (280 of 8: 114.3 -> 100.4), and past that nothing does (halving 440 row tiles
+// 110.5 -> 116 us, 515 175 -> 187).
 // `after`: wide items that the same workgroups draw once their tiles are done (a down stage). There
 // the split goes on only while every item still has a workgroup of its own: past that the tile
 // items and the wide items, which ran side by side, run one after the other (92 wide items and 59
@@ -497,11 +499,18 @@ inline TilePlan tile_plan(uint32_t k, uint32_t n_out) {
 // 8, Q8_0: 64.5 as 131, 81.0 as 262). A gate/up stage draws its tiles behind the wide items, and
 // shorter ones fill its end better (216 wide items and 51 row tiles: 81.6 us as 102 items, 63.0 as
 // 204).
-__device__ __forceinline__ uint32_t split_npi(uint32_t tiles, uint32_t n_ntiles, uint32_t npi, uint32_t after) {
-    while (npi > 1u) {
-        const uint32_t half = (npi + 1u) >> 1, items = tiles * ((n_ntiles + npi - 1u) / npi);
-        if (after == 0u ? items >= gridDim.x : tiles * ((n_ntiles + half - 1u) / half) + after > gridDim.x) break;
+__device__ __forceinline__ uint32_t split_npi(uint32_t tiles, uint32_t n_ntiles, uint32_t npi, uint32_t after,
+                                              uint32_t& n_chunks) {
+    const uint32_t G = gridDim.x;
+    n_chunks = (n_ntiles + npi - 1u) / npi;
+    while (npi > 1u && tiles * n_chunks <= 2u * G) {
+        const uint32_t half = (npi + 1u) >> 1, half_chunks = (n_ntiles + half - 1u) / half;
+        const uint32_t items = tiles * n_chunks, half_items = tiles * half_chunks;
+        const uint32_t rounds = items > G ? 2u : 1u;
+        const uint32_t half_rounds = half_items > 3u * G ? 4u : half_items > 2u * G ? 3u : half_items > G ? 2u : 1u;
+        if (after == 0u ? half_rounds * (half + 2u) >= rounds * (npi + 2u) : half_items + after > G) break;
         npi = half;
+        n_chunks = half_chunks;
     }
     return npi;
 }
@@ -554,7 +563,8 @@ __device__ __forceinline__ void tile_items(const RoutedGemm& g, TileSmem<Frag, N
     auto& sa = sm.sa;
     auto& sw = sm.sw;
     uint32_t* s_dst = sm.s_dst;
-    const uint32_t npi = split_npi(s_pref[512], n_ntiles, npi_launch, after), n_chunks = (n_ntiles + npi - 1u) / npi;
+    uint32_t n_chunks;
+    const uint32_t npi = split_npi(s_pref[512], n_ntiles, npi_launch, after, n_chunks);
     const uint32_t items = s_pref[512] * n_chunks;
     const uint32_t per = (items + 7u) >> 3, x = blockIdx.x & 7u, P = gridDim.x >> 3;
     const uint32_t i_end = (x + 1u) * per < items ? (x + 1u) * per : items;
