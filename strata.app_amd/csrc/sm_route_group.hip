@@ -476,8 +476,12 @@ __global__ __launch_bounds__(kScanThreads) void group_scan_plan_kernel(uint32_t*
 // every entry's slot from them anyway, writes src and dst (its SCATTER form) instead of a
 // scatter launch. One scan carries count and group index, another tiles and misses.
 // The grouping's launches (events) at 1, 4, 21 and 80 tiles: 11.9 -> 6.0, 13.2 -> 6.0, 13.1 -> 8.9
-// and 14.2 -> 9.6 us, the gather unchanged within 0.4 us. 80 tiles is what a thread's registers
-// hold (40 counts each); longer columns are scanned by E / 32 workgroups.
+// and 14.2 -> 9.6 us. The gather grows by its scattered stores, most where it also carries a full
+// layer's checks over narrow rows; grouping and checked gather together (events): 400 tokens of
+// 512 experts (d 2048) 27.0 -> 18.4, 1600 of 256 (4096) 39.4 -> 35.0, 800 of 64 (1024)
+// 23.7 -> 23.3, 1600 of 64 25.1 -> 26.4, with one launch fewer: route and gather of the last two
+// back to back 27.2 -> 22.4 and 29.0 -> 25.1. 80 tiles is what a thread's registers hold (40 counts
+// each); longer columns are scanned by E / 32 workgroups.
 template <uint32_t HELD>
 __global__ __launch_bounds__(kScanThreads) void group_plan_kernel(uint32_t* __restrict__ hist, uint32_t E, uint32_t N,
                                                                   uint32_t n_tiles, Plan* __restrict__ plan,
