@@ -36,6 +36,9 @@ def _cases(layer, moe):
         "split_items": C("tiles_split", 256, 1280, 128, 8, 512, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=306),
         # the same on the streamed path: 2 column tiles per item at the launch, split to 1
         "split_stream": C("tiles_split_s", 128, 1024, 32, 4, 1024, 0, moe.Q2_K, moe.Q4_K, moe.F16, seed=307),
+        # about 275 row tiles x 6 down column tiles: two rounds of items on 256 workgroups become
+        # three of half the length
+        "split_rounds": C("tiles_split_r", 140, 1536, 280, 8, 256, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=308),
         # 512 gate/up items (128 groups x 4 column tiles) on at most 256 workgroups: each
         # workgroup runs items back to back, the next one's copies issued by the current one
         "many_items": C("tiles_many", 1024, 1280, 128, 8, 512, 0, moe.Q4_K, moe.Q8_0, moe.F16, seed=305),
@@ -43,7 +46,7 @@ def _cases(layer, moe):
 
 
 @pytest.mark.parametrize("case", ["q4k_5slab", "q2k_q80", "q80_2slab", "odd_tiles", "split_items",
-                                  "split_stream"])
+                                  "split_stream", "split_rounds"])
 def test_tile_kernels_layer(moe, layer, orc, gpu_ctx, stream, case):
     cfg = _cases(layer, moe)[case]
     print(f"case tiles {case}: T {cfg.rows} d {cfg.hidden} E {cfg.n_experts} top-{cfg.top_k} "
